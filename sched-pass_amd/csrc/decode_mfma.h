@@ -1,7 +1,8 @@
 // decode_mfma.h -- the GQA decode kernel on the CDNA4 matrix cores:
 // bf16 or fp8-e4m3fn KV with bf16 Q, or fp16 KV with fp16 Q (F16), head dim
-// 128, pages of 16..256 tokens, up to 16 q-heads per kv-head (one MFMA
-// column block); and the linear contraction over the same V stream (LINEAR:
+// 128 (64 too for 16-bit caches: half the QK steps and dim blocks below),
+// pages of 16..256 tokens, up to 16 q-heads per kv-head (one MFMA column
+// block); and the linear contraction over the same V stream (LINEAR:
 // no K, weights as MFMA column 0).
 //
 // Layout it reads (one (page, kv-head) chunk each for K and V):
@@ -29,6 +30,14 @@
 // block's A operand is two v_perm_b32 of the lane's own registers; the state
 // goes to LDS with that dim order undone (bf16_vt_operand, fp8_vt_operands,
 // VT).
+//
+// Head dim 64 (16-bit caches): the same tiles with two QK steps and four dim
+// blocks. A lane's token-major V piece is then 8 bytes (vt_operand64), and p
+// is carried in full through the matrix cores (compute_page). HBM-bound as
+// head dim 128 is, at half the bytes per page, so the ring holds twice the
+// pages: 48 requests of 200..2900 tokens, 32 / 8 heads, bf16: 170 us on the
+// VALU kernel, 46 us here (3.5 TB/s; the longest requests end late), with an
+// fp32 output's error against 64 bits at 2.3e-7 (VALU: 3.4e-7).
 //
 // Pages of 32..256 tokens (PG): the kernel streams 16-token blocks; block b
 // is sub-block b % m of table entry b / m (m = page / 16). A d-major V row
@@ -65,13 +74,13 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4_t;
 typedef __attribute__((ext_vector_type(2))) unsigned u32x2_t;
 
-template <bool FP8> struct PageRegs;
-template <> struct PageRegs<false> {
-  u32x4_t k[4]; // 4 x 8 bf16 K
-  u32x4_t v[4]; // V row halves, see bf16_v_operands
-  float lw[4];  // linear mode: the lane's token weights, loaded with the page
+template <bool FP8, int D> struct PageRegs {
+  u32x4_t k[D / 32]; // D / 32 x 8 bf16 K
+  u32x4_t v[D / 32]; // V row halves, see bf16_v_operands (token-major d 64: two
+                     // tokens' 4 dims each, see vt_operand64)
+  float lw[4];       // linear mode: the lane's token weights, loaded with the page
 };
-template <> struct PageRegs<true> {
+template <> struct PageRegs<true, 128> {
   u32x4_t k[2]; // 2 x 16 fp8 K
   u32x4_t v[2]; // V rows lane and lane + 64 (16 fp8 tokens each), see fp8_v_operands
   float lw[4];   // linear mode: the lane's token weights, loaded with the page
@@ -213,9 +222,9 @@ __device__ __forceinline__ void fp8_v_operands(const u32x4_t v[2], unsigned out[
 // for the even rows' second, after which every lane holds its own slice
 // (tokens 4*g4..+3) of both blocks: four 16-byte loads and eight swaps per
 // page instead of eight 8-byte loads.
-__device__ __forceinline__ void bf16_v_operands(u32x4_t v[4]) {
+template <int N> __device__ __forceinline__ void bf16_v_operands(u32x4_t (&v)[N]) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < N; ++i) {
     const auto a = __builtin_amdgcn_permlane16_swap(v[i].x, v[i].z, false, false);
     const auto b = __builtin_amdgcn_permlane16_swap(v[i].y, v[i].w, false, false);
     v[i] = u32x4_t{a[0], b[0], a[1], b[1]}; // (block 2i slice, block 2i + 1 slice)
@@ -230,6 +239,17 @@ __device__ __forceinline__ s16x4_t bf16_vt_operand(const u32x4_t r[4], int blk) 
   const int dw = blk >> 1;
   const unsigned lo = __builtin_amdgcn_perm(r[1][dw], r[0][dw], sel);
   const unsigned hi = __builtin_amdgcn_perm(r[3][dw], r[2][dw], sel);
+  return __builtin_bit_cast(s16x4_t, u32x2_t{lo, hi});
+}
+
+// Token-major 16-bit V of head dim 64: a lane holds dims 4*c16..+3 of tokens
+// 4*g4 + t (8-byte loads), v[t >> 1] dwords 2*(t & 1), 2*(t & 1) + 1. The A
+// operand of block blk is dim 4*c16 + blk of the four tokens.
+__device__ __forceinline__ s16x4_t vt_operand64(const u32x4_t v[2], int blk) {
+  const unsigned sel = (blk & 1) ? 0x07060302u : 0x05040100u;
+  const int dw = blk >> 1;
+  const unsigned lo = __builtin_amdgcn_perm(v[0][2 + dw], v[0][dw], sel);
+  const unsigned hi = __builtin_amdgcn_perm(v[1][2 + dw], v[1][dw], sel);
   return __builtin_bit_cast(s16x4_t, u32x2_t{lo, hi});
 }
 
@@ -278,15 +298,15 @@ __device__ __forceinline__ uint32_t block_in_page(const MfmaTask &T, uint32_t pi
     return 0u;
 }
 
-struct MfmaState {
+template <int D> struct MfmaState {
   float m, lsum;
-  f32x4_t acc[8];
-  bf16x8_t qop[4];
+  f32x4_t acc[D / 16];
+  bf16x8_t qop[D / 32];
 };
 
-template <bool FP8, bool NT, bool LINEAR, bool VT, bool PG>
+template <bool FP8, bool NT, bool LINEAR, bool VT, bool PG, int D>
 __device__ __forceinline__ void issue_page(const KParams &P, const MfmaTask &T, int32_t page,
-                                           uint32_t pidx, PageRegs<FP8> &B) {
+                                           uint32_t pidx, PageRegs<FP8, D> &B) {
   if constexpr (LINEAR) {
     // weights of tokens 4*g4..+3 of the page, for the lanes of MFMA column 0;
     // positions past the context are masked later and not read
@@ -308,19 +328,28 @@ __device__ __forceinline__ void issue_page(const KParams &P, const MfmaTask &T, 
   if constexpr (!FP8) {
     if constexpr (!LINEAR)
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
+      for (int kb = 0; kb < D / 32; ++kb)
         B.k[kb] = gload<NT>(reinterpret_cast<const u32x4_t *>(kp + 64 * kb));
-    if constexpr (VT) {
+    if constexpr (VT && D == 64) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const u32x2_t a =
+            gload<NT>(reinterpret_cast<const u32x2_t *>(pb + (2 * t) * T.vrow_bytes + T.vlane));
+        const u32x2_t b = gload<NT>(
+            reinterpret_cast<const u32x2_t *>(pb + (2 * t + 1) * T.vrow_bytes + T.vlane));
+        B.v[t] = u32x4_t{a.x, a.y, b.x, b.y};
+      }
+    } else if constexpr (VT) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         B.v[i] = gload<NT>(reinterpret_cast<const u32x4_t *>(pb + i * T.vrow_bytes + T.vlane));
     } else if constexpr (PG) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < D / 32; ++i)
         B.v[i] = gload<false>(reinterpret_cast<const u32x4_t *>(pb + i * T.vblk + T.vlane));
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < D / 32; ++i)
         B.v[i] = gload<NT>(reinterpret_cast<const u32x4_t *>(vp + 1024 * i));
     }
   } else {
@@ -350,14 +379,14 @@ __device__ __forceinline__ void issue_page(const KParams &P, const MfmaTask &T, 
   }
 }
 
-template <bool FP8, bool VT, bool PG, bool F16>
-__device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T, MfmaState &S,
-                                             const PageRegs<FP8> &B, int32_t page, uint32_t pidx,
+template <bool FP8, bool VT, bool PG, bool F16, int D>
+__device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T, MfmaState<D> &S,
+                                             const PageRegs<FP8, D> &B, int32_t page, uint32_t pidx,
                                              uint32_t g4) {
   // QK
   f32x4_t sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int kb = 0; kb < 4; ++kb) {
+  for (int kb = 0; kb < D / 32; ++kb) {
     bf16x8_t a;
     if constexpr (!FP8) {
       a = __builtin_bit_cast(bf16x8_t, B.k[kb]);
@@ -401,7 +430,7 @@ __device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T
     const float c = __builtin_amdgcn_exp2f(S.m - mnew);
     S.lsum *= c;
 #pragma unroll
-    for (int blk = 0; blk < 8; ++blk)
+    for (int blk = 0; blk < D / 16; ++blk)
       S.acc[blk] *= c;
   }
   S.m = mnew;
@@ -414,11 +443,21 @@ __device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T
   // leave ~1.2e-3 relative error in the output (p is close to 1 for nearly
   // flat scores), so bf16 / fp8 carry p as hi + lo bf16 halves through two
   // MFMAs (~16 bits, the linear mode's split). fp16's 11 bits (~3e-4) are
-  // kept single.
-  u32x2_t pk, pl;
+  // kept single. Head dim 64 carries p in full: three bf16 parts (24 bits),
+  // or fp16 hi + lo (22 bits, an absolute 2^-25 below that), so that its
+  // results stay those of an fp32 p; its pages have half the dim blocks to
+  // multiply, and the matrix cores are mostly idle either way.
+  u32x2_t pk, pl, p3;
   if constexpr (F16) {
     pk.x = pack_f16_rne(p[0], p[1]);
     pk.y = pack_f16_rne(p[2], p[3]);
+    if constexpr (D == 64) {
+      // through scalars: a bit_cast of a vector's element reads element 0
+      const unsigned w0 = pk.x, w1 = pk.y;
+      const f16x2_t h0 = __builtin_bit_cast(f16x2_t, w0), h1 = __builtin_bit_cast(f16x2_t, w1);
+      pl.x = pack_f16_rne(p[0] - (float)h0.x, p[1] - (float)h0.y);
+      pl.y = pack_f16_rne(p[2] - (float)h1.x, p[3] - (float)h1.y);
+    }
   } else {
     float pv[4];
 #pragma unroll
@@ -426,31 +465,41 @@ __device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T
       pv[v] = FP8 ? p[v] * vs : p[v];
     pk.x = pack_bf16_rne(pv[0], pv[1]);
     pk.y = pack_bf16_rne(pv[2], pv[3]);
-    pl.x = pack_bf16_rne(pv[0] - __uint_as_float(pk.x << 16),
-                         pv[1] - __uint_as_float(pk.x & 0xffff0000u));
-    pl.y = pack_bf16_rne(pv[2] - __uint_as_float(pk.y << 16),
-                         pv[3] - __uint_as_float(pk.y & 0xffff0000u));
+    const float r0 = pv[0] - __uint_as_float(pk.x << 16);
+    const float r1 = pv[1] - __uint_as_float(pk.x & 0xffff0000u);
+    const float r2 = pv[2] - __uint_as_float(pk.y << 16);
+    const float r3 = pv[3] - __uint_as_float(pk.y & 0xffff0000u);
+    pl.x = pack_bf16_rne(r0, r1);
+    pl.y = pack_bf16_rne(r2, r3);
+    if constexpr (D == 64) {
+      p3.x = pack_bf16_rne(r0 - __uint_as_float(pl.x << 16),
+                           r1 - __uint_as_float(pl.x & 0xffff0000u));
+      p3.y = pack_bf16_rne(r2 - __uint_as_float(pl.y << 16),
+                           r3 - __uint_as_float(pl.y & 0xffff0000u));
+    }
   }
   const s16x4_t pop = __builtin_bit_cast(s16x4_t, pk);
 
   // PV
   unsigned v8[8];
-  u32x4_t vb[4];
+  u32x4_t vb[D / 32];
   if constexpr (FP8 && VT) {
     fp8_vt_operands(B.v, v8);
   } else if constexpr (FP8) {
     fp8_v_operands(B.v, v8);
   } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < D / 32; ++i)
       vb[i] = B.v[i];
     if constexpr (!VT)
       bf16_v_operands(vb);
   }
 #pragma unroll
-  for (int blk = 0; blk < 8; ++blk) {
+  for (int blk = 0; blk < D / 16; ++blk) {
     s16x4_t a;
-    if constexpr (VT && !FP8)
+    if constexpr (VT && !FP8 && D == 64)
+      a = vt_operand64(vb, blk);
+    else if constexpr (VT && !FP8)
       a = bf16_vt_operand(vb, blk);
     else if constexpr (!FP8)
       a = __builtin_bit_cast(s16x4_t, (blk & 1) ? u32x2_t{vb[blk >> 1].z, vb[blk >> 1].w}
@@ -458,8 +507,10 @@ __device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T
     else
       a = __builtin_bit_cast(s16x4_t, fp8x4_to_bf16x4(v8[blk]));
     S.acc[blk] = mfma_pv<F16>(a, pop, S.acc[blk]);
-    if constexpr (!F16)
-      S.acc[blk] = mfma_pv<false>(a, __builtin_bit_cast(s16x4_t, pl), S.acc[blk]);
+    if constexpr (!F16 || D == 64)
+      S.acc[blk] = mfma_pv<F16>(a, __builtin_bit_cast(s16x4_t, pl), S.acc[blk]);
+    if constexpr (!F16 && D == 64)
+      S.acc[blk] = mfma_pv<false>(a, __builtin_bit_cast(s16x4_t, p3), S.acc[blk]);
   }
 }
 
@@ -467,8 +518,8 @@ __device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T
 // tokens. w enters PV as column 0 of the B operand, split into bf16 hi + lo
 // halves (two MFMAs) so the weights keep ~16 mantissa bits; V is exact.
 template <bool FP8, bool VT, bool PG>
-__device__ __forceinline__ void linear_page(const KParams &P, const MfmaTask &T, MfmaState &S,
-                                            const PageRegs<FP8> &B, int32_t page, uint32_t pidx,
+__device__ __forceinline__ void linear_page(const KParams &P, const MfmaTask &T,
+                                            MfmaState<128> &S, const PageRegs<FP8, 128> &B, int32_t page, uint32_t pidx,
                                             uint32_t c16, uint32_t g4) {
   float vs = 1.f;
   if constexpr (FP8)
@@ -540,15 +591,15 @@ __device__ __forceinline__ int32_t page_id(const KParams &P, const MfmaTask &T, 
 // waves round-robin, so the assignment (and with it every summation order)
 // depends only on the page index, not on how many pages are read: a task whose
 // shed pages are loaded and masked gives the same bits as one that skips them.
-template <bool FP8, int NW, int DEPTH, bool NT, bool LINEAR, bool VT, bool PG, bool F16>
-__device__ __forceinline__ void stream_pages(const KParams &P, const MfmaTask &T, MfmaState &S,
+template <bool FP8, int NW, int DEPTH, bool NT, bool LINEAR, bool VT, bool PG, bool F16, int D>
+__device__ __forceinline__ void stream_pages(const KParams &P, const MfmaTask &T, MfmaState<D> &S,
                                              uint32_t lane, uint32_t g4) {
   const uint32_t span = T.p1 - T.p0;
   const int npg = span > T.w ? (int)((span - T.w + NW - 1) / NW) : 0;
   if (npg <= 0)
     return;
   const int last = npg - 1;
-  PageRegs<FP8> buf[DEPTH];
+  PageRegs<FP8, D> buf[DEPTH];
   int32_t pid[DEPTH], idn[DEPTH];
 #pragma unroll
   for (int s = 0; s < DEPTH; ++s) {
@@ -561,14 +612,14 @@ __device__ __forceinline__ void stream_pages(const KParams &P, const MfmaTask &T
   auto pidx_of = [&](int j) __attribute__((always_inline)) { return T.p0 + T.w + NW * (uint32_t)j; };
 #pragma unroll
   for (int s = 0; s < DEPTH; ++s)
-    issue_page<FP8, NT, LINEAR, VT, PG>(P, T, pid[s], pidx_of(min(s, last)), buf[s]);
+    issue_page<FP8, NT, LINEAR, VT, PG, D>(P, T, pid[s], pidx_of(min(s, last)), buf[s]);
 
   auto compute = [&](int s, int j) __attribute__((always_inline)) {
     const uint32_t pidx = pidx_of(j);
     if constexpr (LINEAR)
       linear_page<FP8, VT, PG>(P, T, S, buf[s], pid[s], pidx, lane & 15u, g4);
     else
-      compute_page<FP8, VT, PG, F16>(P, T, S, buf[s], pid[s], pidx, g4);
+      compute_page<FP8, VT, PG, F16, D>(P, T, S, buf[s], pid[s], pidx, g4);
   };
   int j = 0;
   for (; j + 2 * DEPTH <= npg; j += DEPTH) {
@@ -576,7 +627,7 @@ __device__ __forceinline__ void stream_pages(const KParams &P, const MfmaTask &T
     for (int s = 0; s < DEPTH; ++s) {
       compute(s, j + s);
       pid[s] = idn[s];
-      issue_page<FP8, NT, LINEAR, VT, PG>(P, T, pid[s], pidx_of(j + DEPTH + s), buf[s]);
+      issue_page<FP8, NT, LINEAR, VT, PG, D>(P, T, pid[s], pidx_of(j + DEPTH + s), buf[s]);
       idn[s] = page_id<NW, PG>(P, T, min(j + 2 * DEPTH + s, last));
     }
   }
@@ -587,7 +638,7 @@ __device__ __forceinline__ void stream_pages(const KParams &P, const MfmaTask &T
         compute(s, j + s);
         if (j + DEPTH + s < npg) {
           pid[s] = idn[s];
-          issue_page<FP8, NT, LINEAR, VT, PG>(P, T, pid[s], pidx_of(j + DEPTH + s), buf[s]);
+          issue_page<FP8, NT, LINEAR, VT, PG, D>(P, T, pid[s], pidx_of(j + DEPTH + s), buf[s]);
         }
       }
     }
@@ -685,25 +736,28 @@ __device__ __forceinline__ void append_token_fp8(const KParams &P, uint32_t r, u
 // An urgent task's stream at the launch's ring depth: any depth in
 // [DLO, DHI] the host accepted (SchedDecodeArgs.pf_dist); 0 = DHI. Every
 // depth computes the same pages in the same order, so the bits do not change.
-template <bool FP8, int NW, int DLO, int DHI, bool NT, bool LINEAR, bool VT, bool PG, bool F16>
-__device__ __forceinline__ void stream_urgent(const KParams &P, const MfmaTask &T, MfmaState &S,
+template <bool FP8, int NW, int DLO, int DHI, bool NT, bool LINEAR, bool VT, bool PG, bool F16,
+          int D>
+__device__ __forceinline__ void stream_urgent(const KParams &P, const MfmaTask &T,
+                                              MfmaState<D> &S,
                                               uint32_t lane, uint32_t g4) {
   if constexpr (DLO < DHI) {
     if (P.pf_depth == (uint32_t)DLO) {
-      stream_pages<FP8, NW, DLO, NT, LINEAR, VT, PG, F16>(P, T, S, lane, g4);
+      stream_pages<FP8, NW, DLO, NT, LINEAR, VT, PG, F16, D>(P, T, S, lane, g4);
       return;
     }
-    stream_urgent<FP8, NW, DLO + 1, DHI, NT, LINEAR, VT, PG, F16>(P, T, S, lane, g4);
+    stream_urgent<FP8, NW, DLO + 1, DHI, NT, LINEAR, VT, PG, F16, D>(P, T, S, lane, g4);
   } else {
-    stream_pages<FP8, NW, DHI, NT, LINEAR, VT, PG, F16>(P, T, S, lane, g4);
+    stream_pages<FP8, NW, DHI, NT, LINEAR, VT, PG, F16, D>(P, T, S, lane, g4);
   }
 }
 
 template <bool FP8, int NW, int GMAX, int DEPTH_S, int DEPTH_U, bool LINEAR = false,
-          bool VT = false, bool PG = false, bool F16 = false>
+          bool VT = false, bool PG = false, bool F16 = false, int D = 128>
 __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
   static_assert(!(F16 && (FP8 || LINEAR)), "fp16: softmax over an fp16 cache");
-  __shared__ float s_acc[NW][GMAX][128];
+  static_assert(D == 128 || (D == 64 && !FP8 && !LINEAR), "head dim 64: softmax, 16-bit cache");
+  __shared__ float s_acc[NW][GMAX][D];
   __shared__ float s_m[NW][GMAX];
   __shared__ float s_l[NW][GMAX];
   const uint32_t lane = threadIdx.x & 63u;
@@ -750,7 +804,7 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
     }
     T.w = w;
     bool wrote = false; // this wave stored the step's token (fused append)
-    if constexpr (!LINEAR && VT) {
+    if constexpr (!LINEAR && VT && D == 128) {
       // fused append: the item holding the new token writes it (in the
       // wave that streams its page) before streaming. A stale plan may hold
       // no item for that page; then chunk 0's item writes it too, so the
@@ -785,14 +839,14 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
     }
     T.kbase = static_cast<const uint8_t *>(P.k_pool) + (int64_t)c16 * P.kts * EB + 16u * g4;
     // fp8: whole row 16*g4 + c16; bf16: half g4/2 of row 16*(g4%2) + c16;
-    // token-major: dims 8*c16.. of token 4*g4 (then rows 4*g4 + 1..3)
+    // token-major: dims D/16 * c16.. of token 4*g4 (then rows 4*g4 + 1..3)
     T.vbase = static_cast<const uint8_t *>(P.v_pool) +
-              (VT ? (int64_t)(4u * g4) * P.vts * EB + 8u * EB * c16
+              (VT ? (int64_t)(4u * g4) * P.vts * EB + D / 16 * EB * c16
                : FP8 ? (int64_t)(c16 + 16u * g4) * P.vds
                      : (int64_t)(c16 + 16u * (g4 & 1u)) * P.vds * EB + 16u * (g4 >> 1));
     T.vrow_bytes = P.vts * EB;
     if constexpr (VT)
-      T.vlane = (uint32_t)(4u * g4 * (uint32_t)T.vrow_bytes + 8u * EB * c16);
+      T.vlane = (uint32_t)(4u * g4 * (uint32_t)T.vrow_bytes + D / 16 * EB * c16);
     else
       T.vlane = (uint32_t)(T.vbase - static_cast<const uint8_t *>(P.v_pool));
     T.ksub = 16 * P.kts * EB;
@@ -803,16 +857,16 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
     T.vpage_bytes = P.vps * EB;
     T.vhead_bytes = P.vhs * EB * T.h;
 
-    MfmaState S;
+    MfmaState<D> S;
     S.m = kMInit;
     S.lsum = 0.f;
 #pragma unroll
-    for (int blk = 0; blk < 8; ++blk)
+    for (int blk = 0; blk < D / 16; ++blk)
       S.acc[blk] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const uint32_t G = LINEAR ? 1u : P.G;
-    const int64_t qrow = ((int64_t)T.r * P.Hq + T.h * G + c16) * 128;
+    const int64_t qrow = ((int64_t)T.r * P.Hq + T.h * G + c16) * D;
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
+    for (int kb = 0; kb < D / 32; ++kb) {
       u32x4_t qv = {0u, 0u, 0u, 0u};
       if (!LINEAR && c16 < G) {
         const uint32_t d0 = qk_dim(FP8, kb, g4);
@@ -836,13 +890,13 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
     if (wrote)
       __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
     if ((T.p1 - T.p0 > kLongItemPages || (kLateDeep && last_round)) && !pol.polite)
-      stream_pages<FP8, NW, DEPTH_U, false, LINEAR, VT, PG, F16>(P, T, S, lane, g4);
+      stream_pages<FP8, NW, DEPTH_U, false, LINEAR, VT, PG, F16, D>(P, T, S, lane, g4);
     else if (pol.urgent)
-      stream_urgent<FP8, NW, DEPTH_S, DEPTH_U, kStockNT, LINEAR, VT, PG, F16>(P, T, S, lane, g4);
+      stream_urgent<FP8, NW, DEPTH_S, DEPTH_U, kStockNT, LINEAR, VT, PG, F16, D>(P, T, S, lane, g4);
     else if (pol.polite)
-      stream_pages<FP8, NW, DEPTH_S, true, LINEAR, VT, PG, F16>(P, T, S, lane, g4);
+      stream_pages<FP8, NW, DEPTH_S, true, LINEAR, VT, PG, F16, D>(P, T, S, lane, g4);
     else
-      stream_pages<FP8, NW, DEPTH_S, kStockNT, LINEAR, VT, PG, F16>(P, T, S, lane, g4);
+      stream_pages<FP8, NW, DEPTH_S, kStockNT, LINEAR, VT, PG, F16, D>(P, T, S, lane, g4);
 
     // Wave states to LDS (l summed over the 4 lane rows first), then the
     // work item's result: output, or partial + fixed-order task merge.
@@ -853,23 +907,23 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
         s_l[w][c16] = lt;
       }
       if constexpr (VT) {
-        // row 4*g4 + i of block blk is dim 8*(4*g4 + i) + blk
+        // row 4*g4 + i of block blk is dim D/16 * (4*g4 + i) + blk
 #pragma unroll
-        for (int blk = 0; blk < 8; ++blk)
+        for (int blk = 0; blk < D / 16; ++blk)
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            s_acc[w][c16][8 * (4 * g4 + i) + blk] = S.acc[blk][i];
+            s_acc[w][c16][D / 16 * (4 * g4 + i) + blk] = S.acc[blk][i];
       } else {
 #pragma unroll
-        for (int blk = 0; blk < 8; ++blk)
+        for (int blk = 0; blk < D / 16; ++blk)
           *reinterpret_cast<f32x4_t *>(&s_acc[w][c16][16 * blk + 4 * g4]) = S.acc[blk];
       }
     }
     __syncthreads();
     if (stale)
-      mark_stale<NW, 128, LINEAR>(P, I.chunk, T.r, T.h, G);
+      mark_stale<NW, D, LINEAR>(P, I.chunk, T.r, T.h, G);
     else
-      finish_item<NW, GMAX, 128, float, LINEAR>(P, wi, task, I.chunk, R.nchunks, T.r, T.h, G,
+      finish_item<NW, GMAX, D, float, LINEAR>(P, wi, task, I.chunk, R.nchunks, T.r, T.h, G,
                                                 s_acc, s_m, s_l);
     timer_commit(P.L, toff, task, t0);
   });

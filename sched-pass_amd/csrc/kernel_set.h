@@ -46,6 +46,12 @@
 #define SCHED_PD_MFMA_DEPTH_F16_URGENT 3
 #endif
 
+// Head dim 64 (16-bit caches): half the bytes per page, so twice the pages in
+// flight; one depth (no deeper urgent ring, pf_dist is refused).
+#ifndef SCHED_PD_MFMA_DEPTH_D64
+#define SCHED_PD_MFMA_DEPTH_D64 4
+#endif
+
 namespace schedpd {
 
 constexpr int mfma_ds(bool fp8) { return fp8 ? SCHED_PD_MFMA_DEPTH_FP8 : SCHED_PD_MFMA_DEPTH; }
@@ -97,6 +103,26 @@ constexpr int mfma_du(bool fp8, bool vt, bool pg, bool f16 = false) {
   SCHED_PD_MFMA_SOFTMAX(PRE, false, false, true, true)                                           \
   SCHED_PD_MFMA_SOFTMAX(PRE, false, true, true, true)
 
+// Head dim 64, 16-bit caches, softmax.
+#define SCHED_PD_MFMA_D64_ONE(PRE, GMAX, VT, PG, F16)                                            \
+  PRE template __global__ void schedpd::decode_mfma<false, SCHED_PD_MFMA_NW, GMAX,               \
+                                                    SCHED_PD_MFMA_DEPTH_D64,                     \
+                                                    SCHED_PD_MFMA_DEPTH_D64, false, VT, PG, F16, \
+                                                    64>(schedpd::KParams);
+#define SCHED_PD_MFMA_D64_LAYOUT(PRE, VT, PG, F16)                                               \
+  SCHED_PD_MFMA_D64_ONE(PRE, 4, VT, PG, F16)                                                     \
+  SCHED_PD_MFMA_D64_ONE(PRE, 8, VT, PG, F16)                                                     \
+  SCHED_PD_MFMA_D64_ONE(PRE, 16, VT, PG, F16)
+#define SCHED_PD_MFMA_D64(PRE)                                                                   \
+  SCHED_PD_MFMA_D64_LAYOUT(PRE, false, false, false)                                             \
+  SCHED_PD_MFMA_D64_LAYOUT(PRE, true, false, false)                                              \
+  SCHED_PD_MFMA_D64_LAYOUT(PRE, false, true, false)                                              \
+  SCHED_PD_MFMA_D64_LAYOUT(PRE, true, true, false)                                               \
+  SCHED_PD_MFMA_D64_LAYOUT(PRE, false, false, true)                                              \
+  SCHED_PD_MFMA_D64_LAYOUT(PRE, true, false, true)                                               \
+  SCHED_PD_MFMA_D64_LAYOUT(PRE, false, true, true)                                               \
+  SCHED_PD_MFMA_D64_LAYOUT(PRE, true, true, true)
+
 // VALU kernels: kv element type x head dim, each for 1 / 4 / 16 q-heads per
 // kv-head and the linear mode.
 #define SCHED_PD_VALU_ONE(PRE, KVT, D)                                                           \
@@ -139,6 +165,7 @@ constexpr int mfma_du(bool fp8, bool vt, bool pg, bool f16 = false) {
   SCHED_PD_MFMA_FP8_TOKMAJOR(extern)                                                             \
   SCHED_PD_MFMA_F16(extern)                                                                      \
   SCHED_PD_MFMA_F16_PAGEBLOCKS(extern)                                                           \
+  SCHED_PD_MFMA_D64(extern)                                                                      \
   SCHED_PD_VALU_ALL(extern)                                                                      \
   SCHED_PD_WAVE_ALL(extern)                                                                      \
   SCHED_PD_WAVE_GROUPS(extern)

@@ -77,6 +77,21 @@ template <bool VT, bool PG = false> KernelFn mfma_kernel_f16(uint32_t G) {
   return decode_mfma<false, NW, 16, DS, DU, false, VT, PG, true>;
 }
 
+// Head dim 64: bf16 or fp16 cache, softmax mode.
+template <bool VT, bool PG, bool F16> KernelFn mfma_kernel_d64(uint32_t G) {
+  constexpr int NW = SCHED_PD_MFMA_NW, DS = SCHED_PD_MFMA_DEPTH_D64;
+  if (G <= 4)
+    return decode_mfma<false, NW, 4, DS, DS, false, VT, PG, F16, 64>;
+  if (G <= 8)
+    return decode_mfma<false, NW, 8, DS, DS, false, VT, PG, F16, 64>;
+  return decode_mfma<false, NW, 16, DS, DS, false, VT, PG, F16, 64>;
+}
+template <bool F16> KernelFn mfma_kernel_d64(uint32_t G, bool vt, bool pg) {
+  if (vt)
+    return pg ? mfma_kernel_d64<true, true, F16>(G) : mfma_kernel_d64<true, false, F16>(G);
+  return pg ? mfma_kernel_d64<false, true, F16>(G) : mfma_kernel_d64<false, false, F16>(G);
+}
+
 bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
 uint64_t round256(uint64_t x) { return (x + 255u) & ~uint64_t(255); }
@@ -106,8 +121,12 @@ bool v_token_major(const SchedDecodeArgs *a) {
   return a->v_dim_stride == 1 && a->v_tok_stride != 1;
 }
 
+// Fewest q-heads per kv-head at which the MFMA kernel takes head dim 64 over
+// token-major rows; below it the one-wave kernel.
+constexpr uint32_t kMfmaD64MinGroup = 4;
+
 // The MFMA kernel's shape: bf16/fp8 KV with bf16 Q (or fp16 KV with fp16 Q,
-// softmax), d 128, pages of 16..256 tokens (a power of two), K rows
+// softmax), d 128 (d 64 too for 16-bit KV, softmax), pages of 16..256 tokens (a power of two), K rows
 // dims-contiguous, V d-major rows of one page (or token-major rows),
 // G <= 16, 16-byte aligned pools.
 bool mfma_applies(const SchedDecodeArgs *a) {
@@ -125,8 +144,15 @@ bool mfma_applies(const SchedDecodeArgs *a) {
   }
   const uint32_t G = linear ? 1u : a->num_q_heads / a->num_kv_heads;
   const uint32_t ps = a->page_size;
-  if (a->head_dim != 128 || ps < 16 || ps > 256 || (ps & (ps - 1)) || G > 16)
+  if (ps < 16 || ps > 256 || (ps & (ps - 1)) || G > 16)
     return false;
+  if (a->head_dim == 64) {
+    if (linear || a->kv_dtype == SCHED_PD_FP8_E4M3 ||
+        (v_token_major(a) && G < kMfmaD64MinGroup))
+      return false;
+  } else if (a->head_dim != 128) {
+    return false;
+  }
   const int64_t eb = elem_bytes(a->kv_dtype);
   if (v_token_major(a)) {
     // token rows start 16-byte (16-bit V) or 8-byte (fp8 V) aligned
@@ -146,9 +172,9 @@ bool mfma_applies(const SchedDecodeArgs *a) {
 
 // Ring depths (pages in flight per wave) of the MFMA kernel `a` selects:
 // stock, and the deepest an urgent task may use (its default). 0, 0 for the
-// VALU kernel, which has no ring.
+// VALU kernel, which has no ring, and at head dim 64, whose ring has one depth.
 void ring_depths(const SchedDecodeArgs *a, bool mfma, uint32_t *ds, uint32_t *du) {
-  if (!mfma) {
+  if (!mfma || a->head_dim != 128) { // d 64: one depth, not a caller's choice
     *ds = *du = 0;
     return;
   }
@@ -363,7 +389,10 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel) {
     sel->per_block = SCHED_PD_WAVE_NWT;
   } else if (mfma) {
     const bool pg = a->page_size > 16;
-    if (a->kv_dtype == SCHED_PD_F16)
+    if (a->head_dim == 64)
+      sel->fn = a->kv_dtype == SCHED_PD_F16 ? mfma_kernel_d64<true>(G, v_token_major(a), pg)
+                                            : mfma_kernel_d64<false>(G, v_token_major(a), pg);
+    else if (a->kv_dtype == SCHED_PD_F16)
       sel->fn = v_token_major(a) ? (pg ? mfma_kernel_f16<true, true>(G) : mfma_kernel_f16<true>(G))
                                  : (pg ? mfma_kernel_f16<false, true>(G)
                                        : mfma_kernel_f16<false>(G));
