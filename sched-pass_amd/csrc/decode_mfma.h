@@ -36,7 +36,7 @@
 // is carried in full through the matrix cores (compute_page). HBM-bound as
 // head dim 128 is, at half the bytes per page, so the ring holds twice the
 // pages: 48 requests of 200..2900 tokens, 32 / 8 heads, bf16: 170 us on the
-// VALU kernel, 46 us here (3.5 TB/s; the longest requests end late), with an
+// VALU kernel, 38 us here (4.2 TB/s; the longest requests end late), with an
 // fp32 output's error against 64 bits at 2.3e-7 (VALU: 3.4e-7).
 //
 // Pages of 32..256 tokens (PG): the kernel streams 16-token blocks; block b
@@ -51,6 +51,16 @@
 // the wave states merge in LDS in fixed order. Nothing
 // in the arithmetic depends on scheduling, so pi, the work queue and the
 // prefetch depth leave every output bit unchanged.
+//
+// Launches with no lever table at all (STOCK) run a kernel without them: no
+// claim loop, policy, timer or urgent ring, and K through a uniform base and a
+// 32-bit lane offset. It fits the 168 registers of three waves per SIMD (the
+// lever kernels, with their deep ring, take 217..256: two), so three work
+// items share a CU and one's claim chain and merge hide behind the others'
+// loads. Same pages, same order, same bits. 48 requests of 200..2900 tokens at
+// head dim 64: 46 -> 38 us; 256 ragged fp16 requests (NHD): 48.6 -> 38.4; a
+// fused step over 128-page tiles: 118 -> 97; 64 x 2048 tokens: 83.2 -> 81.8
+// (the K pattern of k_operands included: without it 44.4, 46, 109 and 81).
 //
 // Policy lever: urgent tasks stream with a deeper ring than stock (DEPTH_S
 // pages in flight per wave): the launch's pf_dist, any depth in
@@ -274,19 +284,46 @@ __device__ __forceinline__ void fp8_vt_operands(const u32x4_t v[2], unsigned out
   fp8_vt_transpose(v[0].y, v[0].w, v[1].y, v[1].w, out + 4);
 }
 
+// Whether a kernel loads K as k_operands wants it (else 16 bytes of the
+// lane's own token row per step). Not the lever kernel of 16-bit d-major
+// 16-token pages, whose ring of four pages leaves no registers for it.
+constexpr bool k_exchange(bool fp8, bool vt, bool pg, int d, bool stock) {
+  return stock || fp8 || vt || pg || d == 64;
+}
+
+// K rows: load pair (2j, 2j + 1) of lane (c16, g4) is 16 bytes at column
+// 128*j + 16*g4 + 64*(c16 / 8) of token rows c16 % 8 and c16 % 8 + 8, so one
+// load instruction reads whole 128-byte lines of eight rows (reading 64 bytes of
+// all sixteen, as the operands need, touches every line twice, which the
+// non-temporal loads pay for). The lanes 8 apart then trade: the first operand
+// (columns 128*j + 16*g4) keeps the low lanes' first load and takes the low
+// lanes' second one in the high lanes, the second operand (+64) the reverse.
+template <int N> __device__ __forceinline__ void k_operands(u32x4_t (&k)[N]) {
+  constexpr int kRor8 = 0x128; // DPP row_ror:8
+#pragma unroll
+  for (int j = 0; j < N; j += 2)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int a = (int)k[j][i], b = (int)k[j + 1][i];
+      k[j][i] = (unsigned)__builtin_amdgcn_update_dpp(a, b, kRor8, 0xF, 0xC, false);
+      k[j + 1][i] = (unsigned)__builtin_amdgcn_update_dpp(b, a, kRor8, 0xF, 0x3, false);
+    }
+}
+
 struct MfmaTask {
   uint32_t r, h, n, budget;
   int64_t row; // block-table index of the request's first page
   uint32_t p0, p1; // pages [p0, p1) of the task are read by this work item
   uint32_t w;      // this wave: pages p0 + w, p0 + w + NW, ...
-  const uint8_t *kbase; // K pool bytes + per-lane offset
-  const uint8_t *vbase;
+  const uint8_t *kbase; // K pool bytes (+ the lane's offset, but in the stock kernel)
   int64_t kpage_bytes, khead_bytes, vpage_bytes, vhead_bytes;
   int64_t vrow_bytes; // token-major V: bytes between token rows
-  uint32_t vlane;     // token-major V / PG: this lane's V byte offset in a block
+  uint32_t vlane;     // this lane's V byte offset in a block
   uint32_t bshift, bmask; // PG: 16-token blocks per page = 1 << bshift
   int64_t ksub, vsub;     // PG: bytes from one block of a page to the next
   int64_t vblk;           // PG, d-major V: bytes between the lane's dim blocks
+  int64_t k8;             // bytes between K rows 8 tokens apart
+  uint32_t klane;         // stock kernel: this lane's K byte offset in a block
 };
 
 // Offset of pidx's first token within its page (PG), else 0.
@@ -304,7 +341,7 @@ template <int D> struct MfmaState {
   bf16x8_t qop[D / 32];
 };
 
-template <bool FP8, bool NT, bool LINEAR, bool VT, bool PG, int D>
+template <bool FP8, bool NT, bool KX, bool LINEAR, bool VT, bool PG, int D, bool STOCK>
 __device__ __forceinline__ void issue_page(const KParams &P, const MfmaTask &T, int32_t page,
                                            uint32_t pidx, PageRegs<FP8, D> &B) {
   if constexpr (LINEAR) {
@@ -321,15 +358,18 @@ __device__ __forceinline__ void issue_page(const KParams &P, const MfmaTask &T, 
   const uint32_t sub = PG ? (pidx & T.bmask) : 0u;
   const uint8_t *kp = T.kbase + (int64_t)page * T.kpage_bytes + T.khead_bytes +
                       (PG ? (int64_t)sub * T.ksub : 0);
-  const uint8_t *vp = T.vbase + (int64_t)page * T.vpage_bytes + T.vhead_bytes;
-  // PG and token-major V: a uniform block base + the lane's 32-bit offset
+  if constexpr (STOCK) // kbase is uniform there, the lane's offset 32 bits
+    kp += T.klane;
+  const uint8_t *kp8 = kp + T.k8;
+  // V: a uniform block base + the lane's 32-bit offset
   const uint8_t *pb = static_cast<const uint8_t *>(P.v_pool) + (int64_t)page * T.vpage_bytes +
                       T.vhead_bytes + (PG ? (int64_t)sub * T.vsub : 0);
   if constexpr (!FP8) {
     if constexpr (!LINEAR)
 #pragma unroll
       for (int kb = 0; kb < D / 32; ++kb)
-        B.k[kb] = gload<NT>(reinterpret_cast<const u32x4_t *>(kp + 64 * kb));
+        B.k[kb] = gload<NT>(reinterpret_cast<const u32x4_t *>(
+            KX ? ((kb & 1) ? kp8 : kp) + 128 * (kb >> 1) : kp + 64 * kb));
     if constexpr (VT && D == 64) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
@@ -350,13 +390,13 @@ __device__ __forceinline__ void issue_page(const KParams &P, const MfmaTask &T, 
     } else {
 #pragma unroll
       for (int i = 0; i < D / 32; ++i)
-        B.v[i] = gload<NT>(reinterpret_cast<const u32x4_t *>(vp + 1024 * i));
+        B.v[i] = gload<NT>(reinterpret_cast<const u32x4_t *>(pb + T.vlane + 1024 * i));
     }
   } else {
     if constexpr (!LINEAR)
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc)
-        B.k[cc] = gload<NT>(reinterpret_cast<const u32x4_t *>(kp + 64 * cc));
+        B.k[cc] = gload<NT>(reinterpret_cast<const u32x4_t *>(!KX ? kp + 64 * cc : cc ? kp8 : kp));
     const int64_t si = ((int64_t)page * P.Hkv + T.h) * P.scale_stride;
     B.ks = (!LINEAR && P.k_scale) ? P.k_scale[si] : 1.f;
     B.vs = P.v_scale ? P.v_scale[si] : 1.f;
@@ -373,25 +413,32 @@ __device__ __forceinline__ void issue_page(const KParams &P, const MfmaTask &T, 
       B.v[0] = gload<false>(reinterpret_cast<const u32x4_t *>(pb + T.vlane));
       B.v[1] = gload<false>(reinterpret_cast<const u32x4_t *>(pb + T.vblk + T.vlane));
     } else {
-      B.v[0] = gload<NT>(reinterpret_cast<const u32x4_t *>(vp));
-      B.v[1] = gload<NT>(reinterpret_cast<const u32x4_t *>(vp + 64 * 16));
+      B.v[0] = gload<NT>(reinterpret_cast<const u32x4_t *>(pb + T.vlane));
+      B.v[1] = gload<NT>(reinterpret_cast<const u32x4_t *>(pb + T.vlane + 64 * 16));
     }
   }
 }
 
-template <bool FP8, bool VT, bool PG, bool F16, int D>
+template <bool FP8, bool KX, bool VT, bool PG, bool F16, int D>
 __device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T, MfmaState<D> &S,
                                              const PageRegs<FP8, D> &B, int32_t page, uint32_t pidx,
                                              uint32_t g4) {
   // QK
+  constexpr int NK = FP8 ? 2 : D / 32;
+  u32x4_t kk[NK];
+#pragma unroll
+  for (int i = 0; i < NK; ++i)
+    kk[i] = B.k[i];
+  if constexpr (KX)
+    k_operands(kk);
   f32x4_t sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int kb = 0; kb < D / 32; ++kb) {
     bf16x8_t a;
     if constexpr (!FP8) {
-      a = __builtin_bit_cast(bf16x8_t, B.k[kb]);
+      a = __builtin_bit_cast(bf16x8_t, kk[kb]);
     } else {
-      const u32x4_t raw = B.k[kb >> 1];
+      const u32x4_t raw = kk[kb >> 1];
       const unsigned w0 = (kb & 1) ? raw.z : raw.x, w1 = (kb & 1) ? raw.w : raw.y;
       const u32x2_t lo = fp8x4_to_bf16x4(w0), hi = fp8x4_to_bf16x4(w1);
       const u32x4_t packed = {lo.x, lo.y, hi.x, hi.y};
@@ -591,9 +638,11 @@ __device__ __forceinline__ int32_t page_id(const KParams &P, const MfmaTask &T, 
 // waves round-robin, so the assignment (and with it every summation order)
 // depends only on the page index, not on how many pages are read: a task whose
 // shed pages are loaded and masked gives the same bits as one that skips them.
-template <bool FP8, int NW, int DEPTH, bool NT, bool LINEAR, bool VT, bool PG, bool F16, int D>
+template <bool FP8, int NW, int DEPTH, bool NT, bool LINEAR, bool VT, bool PG, bool F16, int D,
+          bool STOCK = false>
 __device__ __forceinline__ void stream_pages(const KParams &P, const MfmaTask &T, MfmaState<D> &S,
                                              uint32_t lane, uint32_t g4) {
+  constexpr bool KX = k_exchange(FP8, VT, PG, D, STOCK);
   const uint32_t span = T.p1 - T.p0;
   const int npg = span > T.w ? (int)((span - T.w + NW - 1) / NW) : 0;
   if (npg <= 0)
@@ -612,14 +661,14 @@ __device__ __forceinline__ void stream_pages(const KParams &P, const MfmaTask &T
   auto pidx_of = [&](int j) __attribute__((always_inline)) { return T.p0 + T.w + NW * (uint32_t)j; };
 #pragma unroll
   for (int s = 0; s < DEPTH; ++s)
-    issue_page<FP8, NT, LINEAR, VT, PG, D>(P, T, pid[s], pidx_of(min(s, last)), buf[s]);
+    issue_page<FP8, NT, KX, LINEAR, VT, PG, D, STOCK>(P, T, pid[s], pidx_of(min(s, last)), buf[s]);
 
   auto compute = [&](int s, int j) __attribute__((always_inline)) {
     const uint32_t pidx = pidx_of(j);
     if constexpr (LINEAR)
       linear_page<FP8, VT, PG>(P, T, S, buf[s], pid[s], pidx, lane & 15u, g4);
     else
-      compute_page<FP8, VT, PG, F16, D>(P, T, S, buf[s], pid[s], pidx, g4);
+      compute_page<FP8, KX, VT, PG, F16, D>(P, T, S, buf[s], pid[s], pidx, g4);
   };
   int j = 0;
   for (; j + 2 * DEPTH <= npg; j += DEPTH) {
@@ -627,7 +676,7 @@ __device__ __forceinline__ void stream_pages(const KParams &P, const MfmaTask &T
     for (int s = 0; s < DEPTH; ++s) {
       compute(s, j + s);
       pid[s] = idn[s];
-      issue_page<FP8, NT, LINEAR, VT, PG, D>(P, T, pid[s], pidx_of(j + DEPTH + s), buf[s]);
+      issue_page<FP8, NT, KX, LINEAR, VT, PG, D, STOCK>(P, T, pid[s], pidx_of(j + DEPTH + s), buf[s]);
       idn[s] = page_id<NW, PG>(P, T, min(j + 2 * DEPTH + s, last));
     }
   }
@@ -638,7 +687,7 @@ __device__ __forceinline__ void stream_pages(const KParams &P, const MfmaTask &T
         compute(s, j + s);
         if (j + DEPTH + s < npg) {
           pid[s] = idn[s];
-          issue_page<FP8, NT, LINEAR, VT, PG, D>(P, T, pid[s], pidx_of(j + DEPTH + s), buf[s]);
+          issue_page<FP8, NT, KX, LINEAR, VT, PG, D, STOCK>(P, T, pid[s], pidx_of(j + DEPTH + s), buf[s]);
         }
       }
     }
@@ -753,7 +802,8 @@ __device__ __forceinline__ void stream_urgent(const KParams &P, const MfmaTask &
 }
 
 template <bool FP8, int NW, int GMAX, int DEPTH_S, int DEPTH_U, bool LINEAR = false,
-          bool VT = false, bool PG = false, bool F16 = false, int D = 128>
+          bool VT = false, bool PG = false, bool F16 = false, int D = 128, bool STOCK = false>
+__attribute__((amdgpu_waves_per_eu(STOCK ? 3 : 1)))
 __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
   static_assert(!(F16 && (FP8 || LINEAR)), "fp16: softmax over an fp16 cache");
   static_assert(D == 128 || (D == 64 && !FP8 && !LINEAR), "head dim 64: softmax, 16-bit cache");
@@ -765,13 +815,13 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
   // page ids) then stays in SGPRs with uniform branches.
   const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t c16 = lane & 15u, g4 = lane >> 4;
-  const bool toff = timer_off_latched(P.L);
+  const bool toff = STOCK || timer_off_latched(P.L);
   constexpr uint32_t EB = FP8 ? 1u : 2u; // bytes per KV element
 
   run_tasks(P.L, [&](uint32_t wi, bool last_round) __attribute__((always_inline)) {
     if (wi >= P.L.nitems)
       return;
-    const unsigned long long t0 = read_clock(P.L.wallclock);
+    const unsigned long long t0 = STOCK ? 0ull : read_clock(P.L.wallclock);
     const ItemRow I = item_row(P, wi);
     const uint32_t task = I.task;
     if (task >= P.ntasks)
@@ -781,7 +831,8 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
     T.h = task % P.Hkv;
     T.row = P.indptr ? (int64_t)__builtin_amdgcn_readfirstlane(P.indptr[T.r])
                      : (int64_t)T.r * P.bt_stride;
-    const TaskPolicy pol = task_policy(P.L, task);
+    const TaskPolicy pol =
+        STOCK ? TaskPolicy{false, false, 0xFFFFFFFFu} : task_policy(P.L, task);
     T.n = ctx_tokens(P, T.r);
     T.budget = pol.budget;
     const uint32_t ext = load_extent(P, T.n, pol.budget);
@@ -837,18 +888,18 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
         }
       }
     }
-    T.kbase = static_cast<const uint8_t *>(P.k_pool) + (int64_t)c16 * P.kts * EB + 16u * g4;
+    const int64_t klane = k_exchange(FP8, VT, PG, D, STOCK)
+                              ? (int64_t)(c16 & 7u) * P.kts * EB + 16u * g4 + 64u * (c16 >> 3)
+                              : (int64_t)c16 * P.kts * EB + 16u * g4;
+    T.klane = (uint32_t)klane;
+    T.kbase = static_cast<const uint8_t *>(P.k_pool) + (STOCK ? 0 : klane);
+    T.k8 = 8 * P.kts * EB;
     // fp8: whole row 16*g4 + c16; bf16: half g4/2 of row 16*(g4%2) + c16;
     // token-major: dims D/16 * c16.. of token 4*g4 (then rows 4*g4 + 1..3)
-    T.vbase = static_cast<const uint8_t *>(P.v_pool) +
-              (VT ? (int64_t)(4u * g4) * P.vts * EB + D / 16 * EB * c16
-               : FP8 ? (int64_t)(c16 + 16u * g4) * P.vds
-                     : (int64_t)(c16 + 16u * (g4 & 1u)) * P.vds * EB + 16u * (g4 >> 1));
     T.vrow_bytes = P.vts * EB;
-    if constexpr (VT)
-      T.vlane = (uint32_t)(4u * g4 * (uint32_t)T.vrow_bytes + D / 16 * EB * c16);
-    else
-      T.vlane = (uint32_t)(T.vbase - static_cast<const uint8_t *>(P.v_pool));
+    T.vlane = VT    ? 4u * g4 * (uint32_t)T.vrow_bytes + D / 16 * EB * c16
+              : FP8 ? (c16 + 16u * g4) * (uint32_t)P.vds
+                    : (c16 + 16u * (g4 & 1u)) * (uint32_t)P.vds * EB + 16u * (g4 >> 1);
     T.ksub = 16 * P.kts * EB;
     T.vsub = VT ? 16 * P.vts * EB : 16 * (int64_t)EB;
     T.vblk = FP8 ? 64 * P.vds : 32 * P.vds * EB;
@@ -889,7 +940,12 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
     // first (issued before the Q loads above, so their latency overlaps)
     if (wrote)
       __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-    if ((T.p1 - T.p0 > kLongItemPages || (kLateDeep && last_round)) && !pol.polite)
+    if constexpr (STOCK) {
+      if (T.p1 - T.p0 > kLongItemPages)
+        stream_pages<FP8, NW, DEPTH_S, false, LINEAR, VT, PG, F16, D, true>(P, T, S, lane, g4);
+      else
+        stream_pages<FP8, NW, DEPTH_S, kStockNT, LINEAR, VT, PG, F16, D, true>(P, T, S, lane, g4);
+    } else if ((T.p1 - T.p0 > kLongItemPages || (kLateDeep && last_round)) && !pol.polite)
       stream_pages<FP8, NW, DEPTH_U, false, LINEAR, VT, PG, F16, D>(P, T, S, lane, g4);
     else if (pol.urgent)
       stream_urgent<FP8, NW, DEPTH_S, DEPTH_U, kStockNT, LINEAR, VT, PG, F16, D>(P, T, S, lane, g4);
@@ -925,8 +981,9 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
     else
       finish_item<NW, GMAX, D, float, LINEAR>(P, wi, task, I.chunk, R.nchunks, T.r, T.h, G,
                                                 s_acc, s_m, s_l);
-    timer_commit(P.L, toff, task, t0);
-  });
+    if constexpr (!STOCK)
+      timer_commit(P.L, toff, task, t0);
+  }, NoLevers<STOCK>{});
 }
 
 } // namespace schedpd

@@ -52,9 +52,19 @@
 #define SCHED_PD_MFMA_DEPTH_D64 4
 #endif
 
+// The launches without lever tables (decode_mfma's STOCK): fp8 token-major V
+// at depth 4 spills within the 168 registers of three waves per SIMD; 3 fits.
+#ifndef SCHED_PD_MFMA_DEPTH_FP8_VT_STOCK
+#define SCHED_PD_MFMA_DEPTH_FP8_VT_STOCK 3
+#endif
+
 namespace schedpd {
 
 constexpr int mfma_ds(bool fp8) { return fp8 ? SCHED_PD_MFMA_DEPTH_FP8 : SCHED_PD_MFMA_DEPTH; }
+constexpr int mfma_stock(bool fp8, bool vt) {
+  return fp8 ? (vt ? SCHED_PD_MFMA_DEPTH_FP8_VT_STOCK : SCHED_PD_MFMA_DEPTH_FP8)
+             : SCHED_PD_MFMA_DEPTH;
+}
 // Deepest ring (the urgent default). An urgent task's ring depth is any of
 // mfma_ds .. mfma_du (SchedDecodeArgs.pf_dist).
 constexpr int mfma_du(bool fp8, bool vt, bool pg, bool f16 = false) {
@@ -74,7 +84,11 @@ constexpr int mfma_du(bool fp8, bool vt, bool pg, bool f16 = false) {
   PRE template __global__ void schedpd::decode_mfma<FP8, SCHED_PD_MFMA_NW, GMAX,                 \
                                                     schedpd::mfma_ds(FP8),                       \
                                                     schedpd::mfma_du(FP8, VT, PG, F16), LIN, VT, PG, F16>( \
-      schedpd::KParams);
+      schedpd::KParams);                                                                         \
+  PRE template __global__ void schedpd::decode_mfma<FP8, SCHED_PD_MFMA_NW, GMAX,                 \
+                                                    schedpd::mfma_stock(FP8, VT),                \
+                                                    schedpd::mfma_stock(FP8, VT), LIN, VT, PG,   \
+                                                    F16, 128, true>(schedpd::KParams);
 #define SCHED_PD_MFMA_SOFTMAX(PRE, FP8, VT, PG, F16)                                             \
   SCHED_PD_MFMA_ONE(PRE, FP8, 4, false, VT, PG, F16)                                             \
   SCHED_PD_MFMA_ONE(PRE, FP8, 8, false, VT, PG, F16)                                             \
@@ -108,7 +122,11 @@ constexpr int mfma_du(bool fp8, bool vt, bool pg, bool f16 = false) {
   PRE template __global__ void schedpd::decode_mfma<false, SCHED_PD_MFMA_NW, GMAX,               \
                                                     SCHED_PD_MFMA_DEPTH_D64,                     \
                                                     SCHED_PD_MFMA_DEPTH_D64, false, VT, PG, F16, \
-                                                    64>(schedpd::KParams);
+                                                    64>(schedpd::KParams);                       \
+  PRE template __global__ void schedpd::decode_mfma<false, SCHED_PD_MFMA_NW, GMAX,               \
+                                                    SCHED_PD_MFMA_DEPTH_D64,                     \
+                                                    SCHED_PD_MFMA_DEPTH_D64, false, VT, PG, F16, \
+                                                    64, true>(schedpd::KParams);
 #define SCHED_PD_MFMA_D64_LAYOUT(PRE, VT, PG, F16)                                               \
   SCHED_PD_MFMA_D64_ONE(PRE, 4, VT, PG, F16)                                                     \
   SCHED_PD_MFMA_D64_ONE(PRE, 8, VT, PG, F16)                                                     \

@@ -181,9 +181,17 @@ __device__ __forceinline__ void timer_commit(const LeverTables &L, bool off, uin
 #ifndef SCHED_PD_LATE_ROUNDS
 #define SCHED_PD_LATE_ROUNDS 1u
 #endif
-template <class Body>
-__device__ __forceinline__ void run_tasks(const LeverTables &L, Body &&body) {
+// NoLevers<true>: a launch without any of the tables (known on the host), one
+// item per workgroup.
+template <bool V> struct NoLevers {};
+template <class Body, bool STOCK = false>
+__device__ __forceinline__ void run_tasks(const LeverTables &L, Body &&body,
+                                          NoLevers<STOCK> = NoLevers<STOCK>()) {
   const uint32_t pid = blockIdx.x;
+  if constexpr (STOCK) {
+    body(pid, false);
+    return;
+  }
   uint32_t ntasks = 0u;
   if (L.wq) {
     const bool grid1d = gridDim.y == 1 && gridDim.z == 1;

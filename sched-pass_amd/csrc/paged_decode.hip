@@ -51,16 +51,21 @@ template <typename KVT, int D> KernelFn valu_kernel(bool linear, uint32_t G) {
   return decode_valu<KVT, D, 16, false>;
 }
 
+// `stock`: the launch has no lever tables (decode_mfma's STOCK).
 template <bool FP8, bool VT = false, bool PG = false>
-KernelFn mfma_kernel(uint32_t G, bool linear) {
-  constexpr int NW = SCHED_PD_MFMA_NW, DS = mfma_ds(FP8), DU = mfma_du(FP8, VT, PG);
+KernelFn mfma_kernel(uint32_t G, bool linear, bool stock) {
+  constexpr int NW = SCHED_PD_MFMA_NW, DS = mfma_ds(FP8), DU = mfma_du(FP8, VT, PG),
+                D0 = mfma_stock(FP8, VT);
   if (linear)
-    return decode_mfma<FP8, NW, 4, DS, DU, true, VT, PG, false>;
-  if (G <= 4)
-    return decode_mfma<FP8, NW, 4, DS, DU, false, VT, PG, false>;
-  if (G <= 8)
-    return decode_mfma<FP8, NW, 8, DS, DU, false, VT, PG, false>;
-  return decode_mfma<FP8, NW, 16, DS, DU, false, VT, PG, false>;
+    return stock ? decode_mfma<FP8, NW, 4, D0, D0, true, VT, PG, false, 128, true>
+                 : decode_mfma<FP8, NW, 4, DS, DU, true, VT, PG, false>;
+  if (stock)
+    return G <= 4   ? decode_mfma<FP8, NW, 4, D0, D0, false, VT, PG, false, 128, true>
+           : G <= 8 ? decode_mfma<FP8, NW, 8, D0, D0, false, VT, PG, false, 128, true>
+                    : decode_mfma<FP8, NW, 16, D0, D0, false, VT, PG, false, 128, true>;
+  return G <= 4   ? decode_mfma<FP8, NW, 4, DS, DU, false, VT, PG, false>
+         : G <= 8 ? decode_mfma<FP8, NW, 8, DS, DU, false, VT, PG, false>
+                  : decode_mfma<FP8, NW, 16, DS, DU, false, VT, PG, false>;
 }
 
 uint32_t elem_bytes(uint32_t dt) {
@@ -68,28 +73,34 @@ uint32_t elem_bytes(uint32_t dt) {
 }
 
 // fp16 cache with fp16 Q: 16-byte page-16 layouts, softmax mode.
-template <bool VT, bool PG = false> KernelFn mfma_kernel_f16(uint32_t G) {
-  constexpr int NW = SCHED_PD_MFMA_NW, DS = mfma_ds(false), DU = mfma_du(false, VT, PG, true);
-  if (G <= 4)
-    return decode_mfma<false, NW, 4, DS, DU, false, VT, PG, true>;
-  if (G <= 8)
-    return decode_mfma<false, NW, 8, DS, DU, false, VT, PG, true>;
-  return decode_mfma<false, NW, 16, DS, DU, false, VT, PG, true>;
+template <bool VT, bool PG = false> KernelFn mfma_kernel_f16(uint32_t G, bool stock) {
+  constexpr int NW = SCHED_PD_MFMA_NW, DS = mfma_ds(false), DU = mfma_du(false, VT, PG, true),
+                D0 = mfma_stock(false, VT);
+  if (stock)
+    return G <= 4   ? decode_mfma<false, NW, 4, D0, D0, false, VT, PG, true, 128, true>
+           : G <= 8 ? decode_mfma<false, NW, 8, D0, D0, false, VT, PG, true, 128, true>
+                    : decode_mfma<false, NW, 16, D0, D0, false, VT, PG, true, 128, true>;
+  return G <= 4   ? decode_mfma<false, NW, 4, DS, DU, false, VT, PG, true>
+         : G <= 8 ? decode_mfma<false, NW, 8, DS, DU, false, VT, PG, true>
+                  : decode_mfma<false, NW, 16, DS, DU, false, VT, PG, true>;
 }
 
 // Head dim 64: bf16 or fp16 cache, softmax mode.
-template <bool VT, bool PG, bool F16> KernelFn mfma_kernel_d64(uint32_t G) {
+template <bool VT, bool PG, bool F16, bool STOCK> KernelFn mfma_kernel_d64(uint32_t G) {
   constexpr int NW = SCHED_PD_MFMA_NW, DS = SCHED_PD_MFMA_DEPTH_D64;
-  if (G <= 4)
-    return decode_mfma<false, NW, 4, DS, DS, false, VT, PG, F16, 64>;
-  if (G <= 8)
-    return decode_mfma<false, NW, 8, DS, DS, false, VT, PG, F16, 64>;
-  return decode_mfma<false, NW, 16, DS, DS, false, VT, PG, F16, 64>;
+  return G <= 4   ? decode_mfma<false, NW, 4, DS, DS, false, VT, PG, F16, 64, STOCK>
+         : G <= 8 ? decode_mfma<false, NW, 8, DS, DS, false, VT, PG, F16, 64, STOCK>
+                  : decode_mfma<false, NW, 16, DS, DS, false, VT, PG, F16, 64, STOCK>;
 }
-template <bool F16> KernelFn mfma_kernel_d64(uint32_t G, bool vt, bool pg) {
+template <bool F16, bool STOCK> KernelFn mfma_kernel_d64(uint32_t G, bool vt, bool pg) {
   if (vt)
-    return pg ? mfma_kernel_d64<true, true, F16>(G) : mfma_kernel_d64<true, false, F16>(G);
-  return pg ? mfma_kernel_d64<false, true, F16>(G) : mfma_kernel_d64<false, false, F16>(G);
+    return pg ? mfma_kernel_d64<true, true, F16, STOCK>(G)
+              : mfma_kernel_d64<true, false, F16, STOCK>(G);
+  return pg ? mfma_kernel_d64<false, true, F16, STOCK>(G)
+            : mfma_kernel_d64<false, false, F16, STOCK>(G);
+}
+template <bool F16> KernelFn mfma_kernel_d64(uint32_t G, bool vt, bool pg, bool stock) {
+  return stock ? mfma_kernel_d64<F16, true>(G, vt, pg) : mfma_kernel_d64<F16, false>(G, vt, pg);
 }
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
@@ -232,6 +243,15 @@ template <int G> KernelFn wave_kernel_g(const SchedDecodeArgs *a) {
 KernelFn wave_kernel(const SchedDecodeArgs *a) {
   const uint32_t G = a->num_q_heads / a->num_kv_heads;
   return G == 1 ? wave_kernel_g<1>(a) : G == 2 ? wave_kernel_g<2>(a) : wave_kernel_g<3>(a);
+}
+
+// A launch with no lever tables at all (no pi, control block, timer, queue or
+// device slots), whose K token stride keeps a lane's offset in 32 bits.
+bool stock_launch(const SchedDecodeArgs *a, const KParams &kp) {
+  const int64_t kts = a->k_tok_stride * elem_bytes(a->kv_dtype);
+  return kp.L.order == nullptr && kp.L.ctrl == nullptr && kp.L.timer == nullptr &&
+         kp.L.queue == nullptr && kp.L.rt == 0u &&
+         (a->mode == SCHED_PD_LINEAR || (kts >= 0 && kts <= (INT32_MAX - 64) / 16));
 }
 
 // Validate `a`; on success fill *kp (tables resolved) and *sel.
@@ -389,23 +409,25 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel) {
     sel->per_block = SCHED_PD_WAVE_NWT;
   } else if (mfma) {
     const bool pg = a->page_size > 16;
+    const bool stock = stock_launch(a, *kp), vt = v_token_major(a);
     if (a->head_dim == 64)
-      sel->fn = a->kv_dtype == SCHED_PD_F16 ? mfma_kernel_d64<true>(G, v_token_major(a), pg)
-                                            : mfma_kernel_d64<false>(G, v_token_major(a), pg);
+      sel->fn = a->kv_dtype == SCHED_PD_F16 ? mfma_kernel_d64<true>(G, vt, pg, stock)
+                                            : mfma_kernel_d64<false>(G, vt, pg, stock);
     else if (a->kv_dtype == SCHED_PD_F16)
-      sel->fn = v_token_major(a) ? (pg ? mfma_kernel_f16<true, true>(G) : mfma_kernel_f16<true>(G))
-                                 : (pg ? mfma_kernel_f16<false, true>(G)
-                                       : mfma_kernel_f16<false>(G));
+      sel->fn = vt ? (pg ? mfma_kernel_f16<true, true>(G, stock) : mfma_kernel_f16<true>(G, stock))
+                   : (pg ? mfma_kernel_f16<false, true>(G, stock)
+                         : mfma_kernel_f16<false>(G, stock));
     else if (a->kv_dtype != SCHED_PD_BF16)
-      sel->fn = v_token_major(a) ? (pg ? mfma_kernel<true, true, true>(G, linear)
-                                       : mfma_kernel<true, true>(G, linear))
-                : pg ? mfma_kernel<true, false, true>(G, linear)
-                     : mfma_kernel<true>(G, linear);
-    else if (v_token_major(a))
-      sel->fn = pg ? mfma_kernel<false, true, true>(G, linear)
-                   : mfma_kernel<false, true>(G, linear);
+      sel->fn = vt ? (pg ? mfma_kernel<true, true, true>(G, linear, stock)
+                         : mfma_kernel<true, true>(G, linear, stock))
+                : pg ? mfma_kernel<true, false, true>(G, linear, stock)
+                     : mfma_kernel<true>(G, linear, stock);
+    else if (vt)
+      sel->fn = pg ? mfma_kernel<false, true, true>(G, linear, stock)
+                   : mfma_kernel<false, true>(G, linear, stock);
     else
-      sel->fn = pg ? mfma_kernel<false, false, true>(G, linear) : mfma_kernel<false>(G, linear);
+      sel->fn = pg ? mfma_kernel<false, false, true>(G, linear, stock)
+                   : mfma_kernel<false>(G, linear, stock);
     sel->block = SCHED_PD_MFMA_NW * 64;
     sel->mfma = 1;
   } else {

@@ -1,0 +1,59 @@
+"""Launches without lever tables run the MFMA kernel's lever-free form (three
+waves per SIMD, K lines read whole): the same bits as the lever form, which a
+launch with a timer row runs, and the oracle's values within 16-bit output
+rounding (2^-8 of a row's largest element). Contexts at page, block, wave and
+ring boundaries and on both sides of the long-item line (256 pages)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+import sched_abi as abi
+import sched_pd
+import workloads
+from sched_rt import SchedPlane
+
+pytestmark = pytest.mark.gpu
+
+CTX = [1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 257, 1000, 4096, 4097, 4500]
+
+
+@pytest.mark.parametrize("kv,q", [(torch.bfloat16, torch.bfloat16),
+                                  (torch.float16, torch.float16),
+                                  (torch.float8_e4m3fn, torch.bfloat16)])
+@pytest.mark.parametrize("layout", ["tokmajor", "dmajor"])
+@pytest.mark.parametrize("ps", [16, 64])
+@pytest.mark.parametrize("form", ["softmax", "linear", "tiles"])
+def test_stock_and_lever_forms_agree(schedlib, kv, q, layout, ps, form):
+    if form == "linear" and kv == torch.float16:
+        pytest.skip("no MFMA linear mode over fp16")
+    hkv, G, d = 2, 5, 128
+    b = workloads.make_batch(np.asarray(CTX), num_q_heads=G * hkv, num_kv_heads=hkv, head_dim=d,
+                             page_size=ps, kv_dtype=kv, q_dtype=q, seed=ps, device="cuda")
+    v = b["v_pool"]
+    if layout == "tokmajor":
+        v = v.permute(0, 1, 3, 2).contiguous()
+    kw = dict(v_layout=layout, k_scale=b.get("k_scale"), v_scale=b.get("v_scale"))
+    rows = G * hkv
+    if form == "linear":
+        g = torch.Generator(device="cuda").manual_seed(ps)
+        kw.update(mode=abi.LINEAR, lin_w=torch.rand(max(CTX), device="cuda", generator=g))
+        rows = hkv
+    if form == "tiles":
+        tp = 256 // ps
+        kw.update(tiles=sched_pd.plan_tiles_host(np.asarray(CTX), ps, tp, hkv), tile_pages=tp)
+    outs = []
+    for plane in (None, SchedPlane(max_tasks=len(CTX) * hkv)):
+        out = torch.full((len(CTX), rows, d), 7.0, device="cuda")
+        a = sched_pd.build_args(b["q"], b["k_pool"], v, b["block_table"], b["ctx_lens"], out=out,
+                                plane=plane, **kw)
+        assert sched_pd.kernel_kind(a) == "mfma"
+        sched_pd.launch(a)
+        torch.cuda.synchronize()
+        outs.append(out.cpu())
+    assert torch.equal(outs[0], outs[1])
+    if form == "softmax":
+        ref = np.asarray(oracle.decode(b["q"], b["k_pool"], v, b["block_table"], b["ctx_lens"],
+                                       **kw), np.float64)
+        err = np.abs(outs[0].double().numpy() - ref).max(-1) / np.abs(ref).max(-1)
+        assert err.max() <= 2 ** -8, err.max()
