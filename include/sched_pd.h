@@ -207,6 +207,10 @@ uint64_t sched_rt_timer_host_va(void);
 #define SCHED_PD_FLAG_NO_WAVE 0x20u     /* do not use the one-wave-per-item kernel (G <= 3):
                                            take the MFMA kernel where it applies, else the
                                            general VALU kernel */
+#define SCHED_PD_FLAG_SPLIT 0x80u       /* with tiles NULL: each task runs as up to num_tiles /
+                                           (requests x kv-heads) work items of tile_pages
+                                           pages or more, cut from the context on the device
+                                           (sched_paged_decode_auto_split fills these in) */
 #define SCHED_PD_FLAG_NO_MFMA 0x40u     /* do not use the MFMA kernel: the one-wave-per-item
                                            kernel where it applies, else the VALU kernel */
 
@@ -324,9 +328,18 @@ int sched_paged_decode(const SchedDecodeArgs *a, void *stream);
  * hipError_t code. */
 int sched_paged_decode_noalloc(const SchedDecodeArgs *a, void *stream);
 
-/* Bytes of workspace a launch with these arguments needs (0 without tiles,
- * or -1 on invalid arguments). */
+/* Bytes of workspace a launch with these arguments needs (0 without tiles or
+ * SCHED_PD_FLAG_SPLIT, or -1 on invalid arguments). */
 int64_t sched_paged_decode_workspace_bytes(const SchedDecodeArgs *a);
+
+/* For a launch without tiles: decide from its shape whether its tasks are split
+ * on the device, and if so set SCHED_PD_FLAG_SPLIT, tile_pages and num_tiles
+ * in *a. max_pages bounds a request's pages; mean_pages is their mean over the
+ * requests, 0 if the caller does not know it. pi, num_tasks, order_size and the
+ * queue still count tasks. Returns the workspace bytes the launch then needs (0:
+ * not split, -1: invalid arguments). No counterpart in the reference. */
+int64_t sched_paged_decode_auto_split(SchedDecodeArgs *a, uint32_t max_pages,
+                                      uint32_t mean_pages);
 
 /* Work items resident per CU for the kernel `a` selects (workgroups per CU,
  * times the tasks a workgroup of the one-wave-per-task kernel runs; 0 =

@@ -285,10 +285,11 @@ __device__ __forceinline__ void fp8_vt_operands(const u32x4_t v[2], unsigned out
 }
 
 // Whether a kernel loads K as k_operands wants it (else 16 bytes of the
-// lane's own token row per step). Not the lever kernel of 16-bit d-major
-// 16-token pages, whose ring of four pages leaves no registers for it.
-constexpr bool k_exchange(bool fp8, bool vt, bool pg, int d, bool stock) {
-  return stock || fp8 || vt || pg || d == 64;
+// lane's own token row per step). Not the lever kernels of head dim 128: their
+// deep rings leave no registers for it (266 of 256 for a 16-bit d-major V),
+// and the fp8 queue launch ran the same with it (331.5 us).
+constexpr bool k_exchange(int d, bool stock) {
+  return stock || d == 64;
 }
 
 // K rows: load pair (2j, 2j + 1) of lane (c16, g4) is 16 bytes at column
@@ -642,7 +643,7 @@ template <bool FP8, int NW, int DEPTH, bool NT, bool LINEAR, bool VT, bool PG, b
           bool STOCK = false>
 __device__ __forceinline__ void stream_pages(const KParams &P, const MfmaTask &T, MfmaState<D> &S,
                                              uint32_t lane, uint32_t g4) {
-  constexpr bool KX = k_exchange(FP8, VT, PG, D, STOCK);
+  constexpr bool KX = k_exchange(D, STOCK);
   const uint32_t span = T.p1 - T.p0;
   const int npg = span > T.w ? (int)((span - T.w + NW - 1) / NW) : 0;
   if (npg <= 0)
@@ -865,6 +866,7 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
       if (P.app_k != nullptr && T.n > 0u) {
         const uint32_t pos = T.n - 1u, pg = pos / P.ps;
         const bool holds =
+            P.split ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
             P.tiles == nullptr ||
             (P.tile_ranged ? pg >= I.p0 && pg < I.p1 : I.chunk == pg / P.tile_pages);
         if (holds || (stale && I.chunk == 0u)) {
@@ -888,7 +890,7 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
         }
       }
     }
-    const int64_t klane = k_exchange(FP8, VT, PG, D, STOCK)
+    const int64_t klane = k_exchange(D, STOCK)
                               ? (int64_t)(c16 & 7u) * P.kts * EB + 16u * g4 + 64u * (c16 >> 3)
                               : (int64_t)c16 * P.kts * EB + 16u * g4;
     T.klane = (uint32_t)klane;

@@ -184,18 +184,24 @@ __device__ __forceinline__ void run_wave_tasks(const LeverTables &L, Body &&body
       const uint32_t Rg = min(R, gridDim.x - g * R);
       v0 = g * R * NWT + w * Rg + j;
     }
-    for (uint32_t v = v0; v < L.nitems; v += gridDim.x * NWT)
-      body(remap_static(L, v, L.nitems));
+    for (uint32_t v = v0; v < L.nitems; v += gridDim.x * NWT) {
+      uint32_t chunk;
+      const uint32_t pos = sub_position(L, v, false, &chunk);
+      body(remap_static(L, pos, L.npi) * L.nsub + chunk);
+    }
     return;
   }
-  const uint32_t W = L.workers;
+  const uint32_t W = L.workers, npos = ntasks;
+  ntasks *= L.nsub;
   if (pid >= W || pid >= ntasks)
     return;
   const uint32_t last_ticket = W + ntasks - 1u;
   const uint32_t lane = threadIdx.x & 63u;
   uint32_t raw = pid;
   while (true) {
-    body(remap_wq(L, raw, ntasks));
+    uint32_t chunk;
+    const uint32_t pos = sub_position(L, raw, true, &chunk);
+    body(remap_wq(L, pos, npos) * L.nsub + chunk);
     uint32_t t = 0u;
     if (lane == 0u) {
       t = __hip_atomic_fetch_add(lt_queue(L), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -296,6 +302,7 @@ __global__ void __launch_bounds__(NWT * 64) decode_wave(KParams P) {
       if (P.app_k != nullptr && n > 0u) {
         const uint32_t pos = n - 1u, pg = pos / ps;
         const bool holds =
+            P.split ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
             P.tiles == nullptr ||
             (P.tile_ranged ? pg >= I.p0 && pg < I.p1 : I.chunk == pg / P.tile_pages);
         if (holds || (stale && I.chunk == 0u)) {

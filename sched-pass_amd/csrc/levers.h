@@ -21,6 +21,9 @@ struct LeverTables {
   uint32_t *queue;           // ticket counter
   uint32_t max_tasks;        // rows in order/ctrl/timer
   uint32_t nitems;           // work items of this launch (static grid size)
+  uint32_t npi;              // positions of pi on the static grid (nitems / nsub)
+  uint32_t nsub;             // items of each position of pi and of the queue (1, or a split
+                             // task's: SCHED_PD_FLAG_SPLIT)
   uint32_t wq;               // 1 = launched as W persistent workers
   uint32_t workers;          // W of a work-queue launch (per-wave kernels)
   uint32_t spread;           // per-wave kernels, static grid: workgroups resident at once
@@ -114,6 +117,25 @@ __device__ __forceinline__ uint32_t remap_wq(const LeverTables &L, uint32_t raw,
   return ok ? mapped : raw;
 }
 
+// With sub-items (L.nsub > 1) pi, num_tasks and the queue's positions are
+// tasks: the task position of grid position or ticket `raw`, and which of its
+// items. On a static grid the first item of every task comes first, so those
+// past a context's end (which only look at its length) come last; a task's
+// items take consecutive tickets.
+__device__ __forceinline__ uint32_t sub_position(const LeverTables &L, uint32_t raw, bool queue,
+                                                 uint32_t *chunk) {
+  *chunk = 0u;
+  if (__builtin_expect(L.nsub <= 1u, 1))
+    return raw;
+  if (queue) {
+    const uint32_t pos = raw / L.nsub;
+    *chunk = raw - pos * L.nsub;
+    return pos;
+  }
+  *chunk = raw / L.npi;
+  return raw - *chunk * L.npi;
+}
+
 // Policy flags and shed budget of one task (reference lib/SchedWeave.cpp:
 // 532-581 and :585-614). Task-uniform: every lane computes the same values
 // from scalar loads.
@@ -188,8 +210,10 @@ template <class Body, bool STOCK = false>
 __device__ __forceinline__ void run_tasks(const LeverTables &L, Body &&body,
                                           NoLevers<STOCK> = NoLevers<STOCK>()) {
   const uint32_t pid = blockIdx.x;
+  uint32_t chunk;
   if constexpr (STOCK) {
-    body(pid, false);
+    const uint32_t pos = sub_position(L, pid, false, &chunk);
+    body(__builtin_amdgcn_readfirstlane(pos * L.nsub + chunk), false);
     return;
   }
   uint32_t ntasks = 0u;
@@ -199,6 +223,8 @@ __device__ __forceinline__ void run_tasks(const LeverTables &L, Body &&body,
     ntasks = armed ? ld_u32(lt_ctrl(L) + SCHED_CTRL_NUM_TASKS_OFF) : 0u;
   }
   const bool queue = ntasks != 0u;
+  const uint32_t npos = ntasks; // what pi and num_tasks count
+  ntasks *= L.nsub;
   if (queue && pid >= ntasks)
     return;
   __shared__ uint32_t s_next;
@@ -221,8 +247,10 @@ __device__ __forceinline__ void run_tasks(const LeverTables &L, Body &&body,
     // with fewer and fewer others beside it
     const bool last_round = queue && ntasks >= 2u * gridDim.x &&
                             raw + SCHED_PD_LATE_ROUNDS * gridDim.x >= ntasks;
-    body(__builtin_amdgcn_readfirstlane(queue ? remap_wq(L, raw, ntasks)
-                                              : remap_static(L, raw, L.nitems)),
+    const uint32_t pos = sub_position(L, raw, queue, &chunk);
+    const uint32_t item =
+        queue ? remap_wq(L, pos, npos) : remap_static(L, pos, L.npi);
+    body(__builtin_amdgcn_readfirstlane(item * L.nsub + chunk),
          last_round);
     if (!queue) {
       raw += gridDim.x;

@@ -338,11 +338,23 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel) {
   }
   kp->ntasks = a->num_requests * a->num_kv_heads;
   kp->L.nitems = kp->ntasks;
-  if (a->tiles) {
-    if (a->tile_format > SCHED_PD_TILES_RANGED)
+  kp->L.nsub = 1u;
+  kp->L.npi = kp->ntasks;
+  const bool split = a->tiles == nullptr && (a->flags & SCHED_PD_FLAG_SPLIT);
+  if (split) {
+    if (kp->ntasks == 0 || a->tile_pages == 0 || a->num_tiles < 2u * kp->ntasks ||
+        a->num_tiles % kp->ntasks)
+      return set_error(hipErrorInvalidValue,
+                       "split tasks need tile_pages > 0 and num_tiles a multiple (2 or more) of "
+                       "the %u tasks", kp->ntasks);
+    kp->split = kp->L.nsub = a->num_tiles / kp->ntasks;
+    kp->split_pages = a->tile_pages;
+  }
+  if (a->tiles || split) {
+    if (a->tiles && a->tile_format > SCHED_PD_TILES_RANGED)
       return set_error(hipErrorInvalidValue, "tile_format %u is not a tile row format",
                        a->tile_format);
-    if (a->num_tiles == 0 || (a->tile_format == SCHED_PD_TILES_PAIRS && a->tile_pages == 0))
+    if (a->num_tiles == 0 || (a->tiles && a->tile_format == SCHED_PD_TILES_PAIRS && a->tile_pages == 0))
       return set_error(hipErrorInvalidValue,
                        "tiles need num_tiles > 0 (and tile_pages > 0 for (task, chunk) rows)");
     const WsLayout W = ws_layout(a);
@@ -355,6 +367,7 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel) {
     kp->tile_pages = a->tile_pages;
     kp->tile_ranged = a->tile_format == SCHED_PD_TILES_RANGED ? 1u : 0u;
     kp->L.nitems = a->num_tiles;
+    kp->L.npi = a->num_tiles / kp->L.nsub;
     kp->ws_stale = reinterpret_cast<uint32_t *>(ws + W.stale_off);
     kp->ws_count = reinterpret_cast<uint32_t *>(ws + W.count_off);
     kp->ws_ml = reinterpret_cast<float *>(ws + W.ml_off);
@@ -528,7 +541,7 @@ int sched_paged_decode_noalloc(const SchedDecodeArgs *a, void *stream) {
     return set_error(hipErrorInvalidValue,
                      "sched_paged_decode_noalloc takes no workspace (it uses the library's "
                      "%llu-byte scratch)", (unsigned long long)kScratchBytes);
-  if (a->tiles == nullptr)
+  if (a->tiles == nullptr && !(a->flags & SCHED_PD_FLAG_SPLIT))
     return sched_paged_decode(a, stream);
   KParams kp;
   Selected sel;
@@ -721,8 +734,70 @@ int64_t sched_paged_decode_workspace_bytes(const SchedDecodeArgs *a) {
   if (a == nullptr || a->num_kv_heads == 0 ||
       (a->mode == SCHED_PD_SOFTMAX && (a->num_q_heads == 0 || a->num_q_heads % a->num_kv_heads)))
     return -1;
-  if (a->tiles == nullptr)
+  if (a->tiles == nullptr && !(a->flags & SCHED_PD_FLAG_SPLIT))
     return 0;
+  return (int64_t)ws_layout(a).total;
+}
+
+// When to split (MFMA, bf16, 8 KB a page; whole -> split, us). A launch of few
+// tasks: chunks of kSplitBytes or more of one kv-head's KV, no more items than
+// kFillItems (16 tasks of 257 pages 57 -> 20; below 1.5 chunks a second item
+// costs more than it saves: fp8, 65 pages in chunks of 64, 15 -> 18), and of
+// kHalfFullTokens or more from half the tasks that fill the chip (256 uniform
+// ones of 129 pages in fours: 43 -> 48). From
+// kFullTasks on only contexts of kLongTokens or more, in four (512 ragged tasks
+// of up to 765 pages 163 -> 126, but of up to 383 pages 71 -> 76: their longest
+// items are better whole). With a page list the mean is known, and chunks
+// follow it (512 ragged fp16 tasks of mean 25 pages: 38 -> 34). The one-wave
+// kernel streams an item on one wave, so its chunks are small (128 tasks of
+// mean 18, at most 69 pages: 34 -> 14), larger once the tasks are many (512
+// uniform ones of 17 pages in fifths: 15 -> 17).
+constexpr uint64_t kSplitBytes = 256u << 10, kWaveSplitBytes = 32u << 10;
+constexpr uint64_t kFillItems = 1024, kFullTasks = 512, kWaveFullTasks = 256, kLongTokens = 8192;
+constexpr uint64_t kHalfFullTokens = 1024;
+// Most items of a launch (the empty ones only look at a length), and of a task
+// (its merge reads them all).
+constexpr uint64_t kMostItems = 2048, kMostChunks = 32;
+
+int64_t sched_paged_decode_auto_split(SchedDecodeArgs *a, uint32_t max_pages,
+                                      uint32_t mean_pages) {
+  KParams kp;
+  Selected sel;
+  if (a == nullptr || prepare(a, &kp, &sel))
+    return -1;
+  const uint64_t ntasks = kp.ntasks;
+  if (a->tiles || ntasks == 0 || max_pages == 0)
+    return 0;
+  const uint64_t page = (uint64_t)a->page_size * a->head_dim * elem_bytes(a->kv_dtype) *
+                        (a->mode == SCHED_PD_LINEAR ? 1u : 2u);
+  const bool wave = sel.mfma == 2;
+  auto pages_of = [&](uint64_t bytes) { return std::max<uint64_t>(1u, bytes / page); };
+  const uint64_t per_item = wave ? kWaveSplitBytes * (ntasks >= kWaveFullTasks ? 4u : 1u)
+                                 : kSplitBytes;
+  uint64_t chunk = std::max<uint64_t>(1u, per_item / page);
+  uint64_t s;
+  if (mean_pages) {
+    chunk = std::max(chunk, std::min<uint64_t>(mean_pages + mean_pages / 4u,
+                                               2u * ntasks * mean_pages / kFillItems));
+    s = (max_pages + chunk - 1u) / chunk;
+  } else if (wave) {
+    s = max_pages / std::max(chunk, ntasks * max_pages / (2u * kFillItems));
+  } else if (ntasks < kFullTasks) {
+    if (ntasks >= kFullTasks / 2u)
+      chunk = std::max<uint64_t>(chunk, kHalfFullTokens / a->page_size);
+    chunk = std::max(chunk, ntasks * max_pages / kFillItems);
+    s = (2u * max_pages + chunk) / (2u * chunk);
+  } else {
+    s = (uint64_t)max_pages * a->page_size >= kLongTokens ? 4u : 1u;
+  }
+  s = std::min(std::min(kMostChunks, (wave ? 4u : 1u) * kMostItems / ntasks), s);
+  if (s < 2u)
+    return 0;
+  if (!mean_pages)
+    chunk = (max_pages + s - 1u) / s;
+  a->flags |= SCHED_PD_FLAG_SPLIT;
+  a->tile_pages = (uint32_t)chunk;
+  a->num_tiles = (uint32_t)(s * ntasks);
   return (int64_t)ws_layout(a).total;
 }
 

@@ -578,7 +578,8 @@ class PagedKvCache:
                 out = torch.empty(len(key), q.shape[1], self.head_dim, dtype=dt,
                                   device=self.device)
             args = sched_pd.build_args(q, self.k_pool, self.v_pool, bt, ctx, out=out,
-                                       k_scale=self.k_scale, v_scale=self.v_scale, **kw)
+                                       k_scale=self.k_scale, v_scale=self.v_scale,
+                                       _auto_split=True, **kw)
             if getattr(self, "_app_indptr", None) is None or \
                     self._app_indptr.numel() != len(key) + 1:
                 self._app_indptr = torch.arange(len(key) + 1, dtype=torch.int32,

@@ -40,6 +40,7 @@ FLAG_CTX_IN_PAGES = 0x8
 FLAG_SHED_LOADS = 0x10
 FLAG_NO_WAVE = 0x20
 FLAG_NO_MFMA = 0x40
+FLAG_SPLIT = 0x80
 TILES_PAIRS, TILES_RANGED = 0, 1
 
 _u32, _f32, _i64, _p = ctypes.c_uint32, ctypes.c_float, ctypes.c_int64, ctypes.c_void_p
@@ -142,6 +143,8 @@ SIGNATURES = {
     "sched_paged_decode_noalloc": (ctypes.c_int, [ctypes.POINTER(SchedDecodeArgs), _p]),
     "sched_paged_decode_occupancy": (ctypes.c_int, [ctypes.POINTER(SchedDecodeArgs)]),
     "sched_paged_decode_workspace_bytes": (ctypes.c_int64, [ctypes.POINTER(SchedDecodeArgs)]),
+    "sched_paged_decode_auto_split": (ctypes.c_int64, [ctypes.POINTER(SchedDecodeArgs),
+                                                       ctypes.c_uint32, ctypes.c_uint32]),
     "sched_paged_decode_kernel_kind": (ctypes.c_int, [ctypes.POINTER(SchedDecodeArgs)]),
     "sched_paged_decode_prefetch_range": (ctypes.c_int, [ctypes.POINTER(SchedDecodeArgs),
                                                          ctypes.POINTER(_u32),

@@ -191,7 +191,7 @@ def upload(a, device) -> torch.Tensor:
     already queued, so a serving loop's host work would never overlap its GPU
     work."""
     t = torch.from_numpy(np.ascontiguousarray(a)) if isinstance(a, np.ndarray) else a
-    dev = torch.device(device)
+    dev = device if isinstance(device, torch.device) else torch.device(device)
     if dev.type != "cuda":
         return t.to(dev)
     if dev.index is None:
@@ -218,6 +218,19 @@ def _need_cuda(t: torch.Tensor, what: str) -> None:
         raise ValueError(f"{what} must be a device tensor (got {t.device})")
 
 
+def _need_int32(t: torch.Tensor, what: str) -> None:
+    if t is not None and (t.dtype != torch.int32 or not t.is_contiguous()):
+        raise ValueError(f"{what} must be contiguous int32")
+
+
+def _raw_stream(stream) -> int:
+    """The handle of `stream`, or of the current device's current stream (read
+    without building the Stream object, 2.5 us of a small call's host time)."""
+    if stream is not None:
+        return stream.cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
 def _on_launch_stream(fn):
     """Run `fn` with its `stream` argument current, so that what it queues
     on the device (uploads of host arrays, workspace clears, the queue
@@ -238,7 +251,8 @@ def build_args(q, k_pool, v_pool, block_table, ctx_lens, *, out,
                tau_scope=abi.TAU_PREFIX, lin_w=None, lin_w_period=0,
                plane=None, rt_tables=False, workers=0, pf_dist=0, flags=0,
                policy=(1.0, 1.0, 0.25), tiles=None, tile_pages=0,
-               workspace=None, check_tables=False, stream=None) -> abi.SchedDecodeArgs:
+               workspace=None, check_tables=False, stream=None,
+               _auto_split=False) -> abi.SchedDecodeArgs:
     """Fill a SchedDecodeArgs from tensors (no launch). With `tiles` (from
     plan_tiles, or a host array from plan_tiles_host or plan_ranges_host,
     which is uploaded here; built from these ctx_lens) long tasks run as
@@ -298,16 +312,20 @@ def build_args(q, k_pool, v_pool, block_table, ctx_lens, *, out,
     a.o_dtype = _dtype_code(out, "out")
     a.out = _ptr(out)
     a.v_pool = _ptr(v_pool)
-    for t, what in ((q, "q"), (k_pool, "k_pool"), (v_pool, "v_pool"), (out, "out"),
-                    (block_table, "block_table"), (ctx_lens, "ctx_lens"),
-                    (page_indptr, "page_indptr"), (k_scale, "k_scale"),
-                    (v_scale, "v_scale"), (lin_w, "lin_w")):
-        if t is not None and not (linear and what in ("q", "k_pool")):
-            _need_cuda(t, what)
-    for t, what in ((block_table, "block_table"), (ctx_lens, "ctx_lens"),
-                    (page_indptr, "page_indptr")):
-        if t is not None and (t.dtype != torch.int32 or not t.is_contiguous()):
-            raise ValueError(f"{what} must be contiguous int32")
+    if not linear:
+        _need_cuda(q, "q")
+        _need_cuda(k_pool, "k_pool")
+    _need_cuda(v_pool, "v_pool")
+    _need_cuda(out, "out")
+    _need_cuda(block_table, "block_table")
+    _need_cuda(ctx_lens, "ctx_lens")
+    _need_cuda(page_indptr, "page_indptr")
+    _need_cuda(k_scale, "k_scale")
+    _need_cuda(v_scale, "v_scale")
+    _need_cuda(lin_w, "lin_w")
+    _need_int32(block_table, "block_table")
+    _need_int32(ctx_lens, "ctx_lens")
+    _need_int32(page_indptr, "page_indptr")
     a.block_table = _ptr(block_table)
     a.ctx_lens = _ptr(ctx_lens)
     if page_indptr is not None:
@@ -386,7 +404,30 @@ def build_args(q, k_pool, v_pool, block_table, ctx_lens, *, out,
     else:
         a.max_tasks = 0
         a.workers = 0
+    if tiles is None and _auto_split and workspace is None:
+        _split_on_device(a, block_table, page_indptr, v_pool.device, stream)
     return a
+
+
+def _split_on_device(a, block_table, page_indptr, device, stream) -> None:
+    """Let the library cut the tasks of a launch without tiles into work items
+    (sched_paged_decode_auto_split), with a workspace of the launch stream. A
+    launch that is being captured gets one of its own, cleared in the graph:
+    graphs captured on one stream may be replayed on several."""
+    if page_indptr is None:
+        longest, mean = block_table.shape[1], 0
+    else:
+        longest = block_table.numel()
+        mean = -(-longest // max(1, a.num_requests))
+    need = abi.load_library().sched_paged_decode_auto_split(ctypes.byref(a), longest, mean)
+    if need <= 0:
+        return      # not split, or arguments the launch will refuse
+    if torch.cuda.is_current_stream_capturing():
+        ws = torch.zeros(need, dtype=torch.uint8, device=device)
+    else:
+        ws = workspace_for(need, device, stream=stream,
+                           count_bytes=WS_COUNTERS_OFF + 4 * a.num_requests * a.num_kv_heads)
+    a.workspace, a.workspace_bytes, a._ws = ws.data_ptr(), ws.numel(), ws
 
 
 _WS = {}
@@ -436,11 +477,14 @@ def workspace_for(nbytes: int, device, count_bytes: int = 0, stream=None) -> tor
     partials right after them, so the zeroed prefix is tracked and cleared
     again when a launch needs more counters (which also clears the stale
     counter)."""
-    dev = torch.device(device)
+    dev = device if isinstance(device, torch.device) else torch.device(device)
     if dev.type == "cuda" and dev.index is None:
         dev = torch.device("cuda", torch.cuda.current_device())
-    s = stream if stream is not None else torch.cuda.current_stream(dev)
-    key = (dev.type, dev.index, int(s.cuda_stream))
+    if dev.type == "cuda" and stream is None:
+        key = (dev.type, dev.index, torch._C._cuda_getCurrentRawStream(dev.index))
+    else:
+        s = stream if stream is not None else torch.cuda.current_stream(dev)
+        key = (dev.type, dev.index, int(s.cuda_stream))
     ent = _WS.get(key)
     if ent is None or ent[0].numel() < nbytes:
         ent = [torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=dev), 0]
@@ -820,8 +864,7 @@ def launch(args: abi.SchedDecodeArgs, stream=None) -> None:
     """Launch one decode step described by `args` on `stream` (default: the
     current torch stream). Raises RuntimeError with the library's message."""
     lib = abi.load_library()
-    s = torch.cuda.current_stream() if stream is None else stream
-    rc = lib.sched_paged_decode(ctypes.byref(args), ctypes.c_void_p(s.cuda_stream))
+    rc = lib.sched_paged_decode(ctypes.byref(args), ctypes.c_void_p(_raw_stream(stream)))
     if rc != 0:
         raise RuntimeError(f"sched_paged_decode failed ({rc}): {abi.last_error()}")
 
@@ -833,9 +876,8 @@ def launch_with_append(args: abi.SchedDecodeArgs, append_args, stream=None) -> N
     fp8 caches with token-major V on the MFMA kernel. Raises RuntimeError with
     the library's message for anything else."""
     lib = abi.load_library()
-    s = torch.cuda.current_stream() if stream is None else stream
     rc = lib.sched_paged_decode_append(ctypes.byref(args), ctypes.byref(append_args),
-                                       ctypes.c_void_p(s.cuda_stream))
+                                       ctypes.c_void_p(_raw_stream(stream)))
     if rc != 0:
         raise RuntimeError(f"sched_paged_decode_append failed ({rc}): {abi.last_error()}")
 
@@ -850,7 +892,7 @@ def paged_decode(q, k_pool, v_pool, block_table, ctx_lens, *, out=None,
         dt = out_dtype or (q.dtype if q is not None else torch.float32)
         out = torch.empty(ctx_lens.numel(), rows, d, dtype=dt, device=v_pool.device)
     args = build_args(q, k_pool, v_pool, block_table, ctx_lens, out=out, mode=mode,
-                      stream=stream, **kw)
+                      stream=stream, _auto_split=True, **kw)
     launch(args, stream)
     return out
 
