@@ -422,15 +422,26 @@ def _split_on_device(a, block_table, page_indptr, device, stream) -> None:
     need = abi.load_library().sched_paged_decode_auto_split(ctypes.byref(a), longest, mean)
     if need <= 0:
         return      # not split, or arguments the launch will refuse
+    counters = WS_COUNTERS_OFF + 4 * a.num_requests * a.num_kv_heads
     if torch.cuda.is_current_stream_capturing():
-        ws = torch.zeros(need, dtype=torch.uint8, device=device)
+        ws = torch.empty(need, dtype=torch.uint8, device=device)
+        ws[:counters].zero_()
     else:
-        ws = workspace_for(need, device, stream=stream,
-                           count_bytes=WS_COUNTERS_OFF + 4 * a.num_requests * a.num_kv_heads)
+        # one per (thread, stream): between a thread's clear and its launch no
+        # other thread's launch on the stream may write the counters' place
+        cache = getattr(_SPLIT_WS, "streams", None)
+        if cache is None or len(cache) > _SPLIT_WS_STREAMS:
+            cache = _SPLIT_WS.streams = {}
+        ws = workspace_for(need, device, stream=stream, count_bytes=counters, _cache=cache)
     a.workspace, a.workspace_bytes, a._ws = ws.data_ptr(), ws.numel(), ws
 
 
 _WS = {}
+# Workspaces of launches split on the device, per thread: dropped with it, and
+# all at once should a thread use more streams than this (each is freed to its own
+# stream, behind the launches that use it).
+_SPLIT_WS = threading.local()
+_SPLIT_WS_STREAMS = 16
 
 
 def check_page_table(block_table, ctx_lens, page_size: int, num_pages: int, *,
@@ -469,7 +480,8 @@ def check_page_table(block_table, ctx_lens, page_size: int, num_pages: int, *,
 WS_COUNTERS_OFF = 256
 
 
-def workspace_for(nbytes: int, device, count_bytes: int = 0, stream=None) -> torch.Tensor:
+def workspace_for(nbytes: int, device, count_bytes: int = 0, stream=None,
+                  _cache=None) -> torch.Tensor:
     """A device workspace of at least `nbytes` whose first `count_bytes` (the
     stale counter and the per-task arrival counters) are zero, cached per
     (device, stream): launches on one stream are ordered, launches on two
@@ -485,11 +497,12 @@ def workspace_for(nbytes: int, device, count_bytes: int = 0, stream=None) -> tor
     else:
         s = stream if stream is not None else torch.cuda.current_stream(dev)
         key = (dev.type, dev.index, int(s.cuda_stream))
-    ent = _WS.get(key)
+    cache = _WS if _cache is None else _cache
+    ent = cache.get(key)
     if ent is None or ent[0].numel() < nbytes:
         ent = [torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=dev), 0]
         ent[1] = ent[0].numel()
-        _WS[key] = ent
+        cache[key] = ent
     need_zero = -(-count_bytes // 256) * 256
     if need_zero > ent[1]:
         ent[0][:need_zero].zero_()

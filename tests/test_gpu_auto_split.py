@@ -120,3 +120,26 @@ def test_csr_table_and_graph_replays(schedlib):
         torch.cuda.synchronize()
         assert torch.equal(out.nan_to_num(9.0), base)
         assert torch.equal(run(pos, kw).nan_to_num(9.0), base)
+
+
+def test_threads_on_one_stream(schedlib):
+    """Launches of several threads' shapes interleave on the default stream: each
+    thread's workspace keeps its counters."""
+    import threading
+    cases = [make(k)[:2] for k in ("bf16", "wave", "valu")]
+    want = [run(pos, kw).nan_to_num(9.0) for pos, kw in cases]
+    bad = []
+
+    def work(i):
+        pos, kw = cases[i]
+        for _ in range(60):
+            out = sched_pd.paged_decode(*pos, out_dtype=torch.float32, **kw)
+            if not torch.equal(out.nan_to_num(9.0), want[i]):
+                bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(cases))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
