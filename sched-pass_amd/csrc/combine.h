@@ -67,6 +67,21 @@ __device__ __forceinline__ bool arrive(uint32_t *count, uint32_t nchunks) {
   return last;
 }
 
+// The same for a task split on the device, whose word holds a bit per chunk (at
+// most 32): pi may name a task twice (an entry out of range falls back to its
+// own position), and a chunk that arrives again must neither complete the task
+// early nor be missing from it. What a second arrival leaves behind is cleared
+// before the next launch with lever tables; without them each chunk runs once.
+__device__ __forceinline__ bool arrive_chunk(uint32_t *mask, uint32_t chunk, uint32_t nchunks) {
+  const uint32_t full = 0xFFFFFFFFu >> (32u - nchunks), bit = 1u << chunk;
+  const uint32_t old =
+      __hip_atomic_fetch_or(mask, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const bool last = old != full && (old | bit) == full;
+  if (last)
+    __hip_atomic_store(mask, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return last;
+}
+
 // The merge of a task's partials, in the work item that completes it: the
 // partials of chunks 0 .. nchunks-1 (work items base .. base + nchunks - 1)
 // read in chunk order, outputs (orow + g) * D + j for g < G (linear: orow * D
@@ -213,7 +228,10 @@ __device__ __forceinline__ void finish_item(const KParams &P, uint32_t wi, uint3
   __syncthreads();
   __shared__ uint32_t s_last;
   if (threadIdx.x == 0)
-    s_last = arrive(P.ws_count + task, nchunks) ? 1u : 0u;
+    s_last = (P.L.nsub > 1u ? arrive_chunk(P.ws_count + task, chunk, nchunks)
+                            : arrive(P.ws_count + task, nchunks))
+                 ? 1u
+                 : 0u;
   __syncthreads();
   if (!s_last)
     return;
@@ -225,7 +243,7 @@ __device__ __forceinline__ void finish_item(const KParams &P, uint32_t wi, uint3
 // following from the context length. Ranged rows (task, chunk | nchunks << 16,
 // p0, p1) carry the task's chunk count and the chunk's page range, so the
 // chunks of one task may differ in size. Without a list, work item = task, or
-// (P.split) item task * split + chunk: the task's pages in up to `split` equal
+// (L.nsub > 1) item task * nsub + chunk: the task's pages in up to `nsub` equal
 // chunks of split_pages or more, so few or ragged tasks spread over the chip
 // with no plan (one request of 8191 tokens, 32 / 8 heads: 73 -> 17 us). The
 // chunk size follows from the context alone, never from a shed budget or the
@@ -236,9 +254,9 @@ struct ItemRow {
 
 __device__ __forceinline__ ItemRow item_row(const KParams &P, uint32_t wi) {
   ItemRow I{wi, 0u, 1u, 0u, 0u};
-  if (__builtin_expect(P.split != 0u, 0)) {
-    I.task = wi / P.split;
-    I.chunk = wi - I.task * P.split;
+  if (__builtin_expect(P.L.nsub > 1u, 0)) {
+    I.task = wi / P.L.nsub;
+    I.chunk = wi - I.task * P.L.nsub;
     return I;
   }
   if (P.tiles == nullptr)
@@ -262,16 +280,16 @@ __device__ __forceinline__ ItemRow item_row(const KParams &P, uint32_t wi) {
 // the npages_load pages of the task that are read at all (n context tokens).
 struct ItemRange {
   uint32_t nchunks, p0, p1;
-  uint32_t cp; // P.split: pages per chunk
+  uint32_t cp; // L.nsub > 1: pages per chunk
 };
 
 __device__ __forceinline__ ItemRange item_range(const KParams &P, const ItemRow &I, uint32_t n,
                                                 uint32_t npages_load) {
-  if (__builtin_expect(P.split != 0u, 0)) {
+  if (__builtin_expect(P.L.nsub > 1u, 0)) {
     // chunks wholly past a budget are skipped (the merge of a masked chunk
     // would add exact zeros)
     ItemRange it;
-    it.cp = max(P.split_pages, ((n + P.ps - 1u) / P.ps + P.split - 1u) / P.split);
+    it.cp = max(P.split_pages, ((n + P.ps - 1u) / P.ps + P.L.nsub - 1u) / P.L.nsub);
     it.nchunks = max(1u, (npages_load + it.cp - 1u) / it.cp);
     it.p0 = min(I.chunk * it.cp, npages_load);
     it.p1 = min(it.p0 + it.cp, npages_load);
@@ -312,7 +330,7 @@ __device__ __forceinline__ ItemRange item_range(const KParams &P, const ItemRow 
 // nchunks), which a running item keeps inside the list.
 __device__ __forceinline__ bool item_skip(const KParams &P, uint32_t wi, const ItemRow &I,
                                          const ItemRange &R) {
-  return (P.split && I.chunk >= R.nchunks) ||
+  return (P.L.nsub > 1u && I.chunk >= R.nchunks) ||
          (P.tiles != nullptr && (I.chunk > wi || I.chunk >= R.nchunks));
 }
 

@@ -866,7 +866,7 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
       if (P.app_k != nullptr && T.n > 0u) {
         const uint32_t pos = T.n - 1u, pg = pos / P.ps;
         const bool holds =
-            P.split ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
+            P.L.nsub > 1u ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
             P.tiles == nullptr ||
             (P.tile_ranged ? pg >= I.p0 && pg < I.p1 : I.chunk == pg / P.tile_pages);
         if (holds || (stale && I.chunk == 0u)) {

@@ -258,7 +258,10 @@ __device__ __forceinline__ void finish_wave_item(const KParams &P, uint32_t wi, 
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   uint32_t last = 0u;
   if (lane == 0u)
-    last = arrive(P.ws_count + task, nchunks) ? 1u : 0u;
+    last = (P.L.nsub > 1u ? arrive_chunk(P.ws_count + task, chunk, nchunks)
+                          : arrive(P.ws_count + task, nchunks))
+               ? 1u
+               : 0u;
   if (__builtin_amdgcn_readfirstlane(last))
     merge_partials<D, float, false>(P, wi - chunk, nchunks, G, orow, lane, 64u);
 }
@@ -302,7 +305,7 @@ __global__ void __launch_bounds__(NWT * 64) decode_wave(KParams P) {
       if (P.app_k != nullptr && n > 0u) {
         const uint32_t pos = n - 1u, pg = pos / ps;
         const bool holds =
-            P.split ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
+            P.L.nsub > 1u ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
             P.tiles == nullptr ||
             (P.tile_ranged ? pg >= I.p0 && pg < I.p1 : I.chunk == pg / P.tile_pages);
         if (holds || (stale && I.chunk == 0u)) {

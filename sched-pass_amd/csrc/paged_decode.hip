@@ -32,6 +32,9 @@ namespace {
 // a power of two).
 constexpr uint32_t kMfmaMinGroup = 1;
 
+// Most chunks of a task split on the device: a bit each in its arrival word.
+constexpr uint64_t kMostChunks = 32;
+
 typedef void (*KernelFn)(KParams);
 
 struct Selected {
@@ -343,11 +346,11 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel) {
   const bool split = a->tiles == nullptr && (a->flags & SCHED_PD_FLAG_SPLIT);
   if (split) {
     if (kp->ntasks == 0 || a->tile_pages == 0 || a->num_tiles < 2u * kp->ntasks ||
-        a->num_tiles % kp->ntasks)
+        a->num_tiles % kp->ntasks || a->num_tiles / kp->ntasks > kMostChunks)
       return set_error(hipErrorInvalidValue,
-                       "split tasks need tile_pages > 0 and num_tiles a multiple (2 or more) of "
+                       "split tasks need tile_pages > 0 and num_tiles a multiple (2 to 32) of "
                        "the %u tasks", kp->ntasks);
-    kp->split = kp->L.nsub = a->num_tiles / kp->ntasks;
+    kp->L.nsub = a->num_tiles / kp->ntasks;
     kp->split_pages = a->tile_pages;
   }
   if (a->tiles || split) {
@@ -757,7 +760,7 @@ constexpr uint64_t kFillItems = 1024, kFullTasks = 512, kWaveFullTasks = 256, kL
 constexpr uint64_t kHalfFullTokens = 1024;
 // Most items of a launch (the empty ones only look at a length), and of a task
 // (its merge reads them all).
-constexpr uint64_t kMostItems = 2048, kMostChunks = 32;
+constexpr uint64_t kMostItems = 2048;
 
 int64_t sched_paged_decode_auto_split(SchedDecodeArgs *a, uint32_t max_pages,
                                       uint32_t mean_pages) {
