@@ -298,7 +298,9 @@ typedef struct SchedDecodeArgs {
    * and zero it to reset), then from byte 256 the per-task arrival counters,
    * then per-work-item partial results. The arrival counters must be zero
    * before the first launch; each launch leaves them zero (a stale task's
-   * counter is never touched). Launches sharing one workspace must not
+   * counter is never touched; a SCHED_PD_FLAG_SPLIT launch whose order may
+   * name a task twice zeroes them with a small kernel behind itself, and a
+   * tile list under such an order may leave them nonzero). Launches sharing one workspace must not
    * overlap (use one workspace per stream). */
   void *workspace;
   uint64_t workspace_bytes;

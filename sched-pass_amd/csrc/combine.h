@@ -70,8 +70,9 @@ __device__ __forceinline__ bool arrive(uint32_t *count, uint32_t nchunks) {
 // The same for a task split on the device, whose word holds a bit per chunk (at
 // most 32): pi may name a task twice (an entry out of range falls back to its
 // own position), and a chunk that arrives again must neither complete the task
-// early nor be missing from it. What a second arrival leaves behind is cleared
-// before the next launch with lever tables; without them each chunk runs once.
+// early nor be missing from it. A bit that a second arrival leaves set would do
+// both to the next launch on the workspace, so a launch with an order clears
+// the words behind itself (launch_decode); without one each chunk runs once.
 __device__ __forceinline__ bool arrive_chunk(uint32_t *mask, uint32_t chunk, uint32_t nchunks) {
   const uint32_t full = 0xFFFFFFFFu >> (32u - nchunks), bit = 1u << chunk;
   const uint32_t old =

@@ -532,6 +532,11 @@ __global__ void zero_words(uint32_t *p, uint32_t n) {
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
     p[i] = 0u;
 }
+void launch_zero_words(uint32_t *p, uint32_t n, void *stream) {
+  const uint32_t blocks = (n + 255u) / 256u;
+  hipLaunchKernelGGL(zero_words, dim3(blocks < 1024u ? blocks : 1024u), dim3(256), 0,
+                     (hipStream_t)stream, p, n);
+}
 
 } // namespace
 
@@ -568,10 +573,7 @@ int sched_paged_decode_noalloc(const SchedDecodeArgs *a, void *stream) {
   if (ptr == nullptr)
     return hipErrorInvalidSymbol;
   // the stale counter and this launch's arrival counters start at zero
-  const uint32_t words = (uint32_t)(W.ml_off / 4u);
-  const uint32_t blocks = (words + 255u) / 256u;
-  hipLaunchKernelGGL(zero_words, dim3(blocks < 1024u ? blocks : 1024u), dim3(256), 0,
-                     (hipStream_t)stream, static_cast<uint32_t *>(ptr), words);
+  launch_zero_words(static_cast<uint32_t *>(ptr), (uint32_t)(W.ml_off / 4u), stream);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess)
     return set_error(e, "scratch clear failed: %s", hipGetErrorString(e));
@@ -666,6 +668,14 @@ static int launch_decode(const SchedDecodeArgs *a, const AppendRows *app, void *
   hipError_t e = hipGetLastError();
   if (e != hipSuccess)
     return set_error(e, "kernel launch failed: %s", hipGetErrorString(e));
+  if (kp.L.nsub > 1u && (kp.L.order != nullptr || kp.L.rt)) {
+    // pi may have named a task twice, whose second run's arrivals stay: the
+    // next launch on this workspace starts from clear words again
+    launch_zero_words(kp.ws_count, kp.ntasks, stream);
+    e = hipGetLastError();
+    if (e != hipSuccess)
+      return set_error(e, "arrival counter clear failed: %s", hipGetErrorString(e));
+  }
   if (a->flags & SCHED_PD_FLAG_RT_TABLES)
     return rt_after_launch(stream);
   return 0;

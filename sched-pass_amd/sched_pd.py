@@ -433,9 +433,6 @@ def _split_on_device(a, block_table, page_indptr, device, stream) -> None:
         if cache is None or len(cache) > _SPLIT_WS_STREAMS:
             cache = _SPLIT_WS.streams = {}
         ws = workspace_for(need, device, stream=stream, count_bytes=counters, _cache=cache)
-        if a.order or a.ctrl or a.flags & abi.FLAG_RT_TABLES:
-            # an order may name a task twice: its second run's arrivals stay
-            ws[:counters].zero_()
     a.workspace, a.workspace_bytes, a._ws = ws.data_ptr(), ws.numel(), ws
 
 

@@ -98,6 +98,48 @@ def test_shed_budgets_loaded_or_skipped(schedlib, kind):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("kind", ["bf16", "wave", "valu"])
+def test_an_order_naming_a_task_twice_leaves_nothing_behind(schedlib, kind):
+    """A permitted order (an entry out of range falls back to its own position)
+    that runs a task twice and another not at all: the launch's other rows are
+    the plain ones, its workspace's arrival words end at zero, and the plain
+    launches after it, of other queries and of shorter contexts (fewer chunks),
+    equal the oracle."""
+    pos, kw, hkv, tol = make(kind)
+    base = run(pos, kw).nan_to_num(9.0)
+    n, rows = len(CTX) * hkv, base.shape[1] // hkv
+    order = np.arange(n, dtype=np.int32)
+    order[1] = 0                    # task 0 (4097 tokens) twice, task 1 never
+    order[-1] = n + 7               # falls back to its position
+    for workers in (0, 3):
+        plane = SchedPlane(max_tasks=n)
+        plane.install_order(torch.from_numpy(order), 0)
+        plane.set_num_tasks(n)
+        plane.push()
+        out = torch.full_like(base, 5.0)
+        sched_pd.paged_decode(*pos, out=out, plane=plane, workers=workers, **kw)
+        torch.cuda.synchronize()
+        out = out.nan_to_num(9.0).view(n, rows, -1)
+        want = base.view(n, rows, -1).clone()
+        want[1] = 5.0
+        assert torch.equal(out, want), workers
+        for ws, zeroed in sched_pd._SPLIT_WS.streams.values():
+            words = ws[sched_pd.WS_COUNTERS_OFF:sched_pd.WS_COUNTERS_OFF + 4 * n]
+            assert not words.any(), workers
+        for shorter in (0, 2000, 3400):
+            ctx = torch.clamp(pos[4] - shorter, min=1).int()
+            q = torch.randn(pos[0].shape, device="cuda",
+                            generator=torch.Generator(device="cuda").manual_seed(shorter))
+            again = (q.to(pos[0].dtype), *pos[1:4], ctx)
+            got = torch.full_like(base, 5.0)
+            sched_pd.paged_decode(*again, out=got, **kw)
+            torch.cuda.synchronize()
+            got = got.cpu().double().numpy()
+            ref = np.asarray(oracle.decode(*again, **kw), np.float64)
+            err = np.linalg.norm(got - ref, axis=-1) / np.linalg.norm(ref, axis=-1)
+            assert err.max() <= tol, (workers, shorter, err.max())
+
+
 def test_csr_table_and_graph_replays(schedlib):
     pos, kw, hkv, tol = make("bf16")
     base = run(pos, kw).nan_to_num(9.0)
