@@ -33,7 +33,8 @@
 //
 // Head dim 64 (16-bit caches): the same tiles with two QK steps and four dim
 // blocks. A lane's token-major V piece is then 8 bytes (vt_operand64), and p
-// is carried in full through the matrix cores (compute_page). HBM-bound as
+// is carried in full through the matrix cores (compute_page); V of masked
+// tokens is selected to 0 (mask_v64: gqa d64 step 34.6 -> 34.9 us). HBM-bound as
 // head dim 128 is, at half the bytes per page, so the ring holds twice the
 // pages: 48 requests of 200..2900 tokens, 32 / 8 heads, bf16: 170 us on the
 // VALU kernel, 38 us here (34 split on the device, 4.7 TB/s), with an
@@ -263,6 +264,26 @@ __device__ __forceinline__ s16x4_t vt_operand64(const u32x4_t v[2], int blk) {
   return __builtin_bit_cast(s16x4_t, u32x2_t{lo, hi});
 }
 
+// Zero the V of the lane's tokens 4*g4 + t that do not count (head dim 64).
+// Token-major: token t is dwords 2*(t & 1), 2*(t & 1) + 1 of v[t >> 1]; d-major
+// operands: half t & 1 of dwords t >> 1 (block 2i) and 2 + (t >> 1) (2i + 1).
+template <bool VT> __device__ __forceinline__ void mask_v64(u32x4_t (&v)[2], const bool (&in)[4]) {
+  if constexpr (VT) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const unsigned m = in[t] ? ~0u : 0u;
+      v[t >> 1][2 * (t & 1)] &= m;
+      v[t >> 1][2 * (t & 1) + 1] &= m;
+    }
+  } else {
+    const unsigned m01 = (in[0] ? 0xffffu : 0u) | (in[1] ? 0xffff0000u : 0u);
+    const unsigned m23 = (in[2] ? 0xffffu : 0u) | (in[3] ? 0xffff0000u : 0u);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      v[i] &= u32x4_t{m01, m23, m01, m23};
+  }
+}
+
 // Token-major fp8 V: lane (c16, g4) holds dims 8*c16..+7 of tokens 4*g4 + t
 // (t = 0..3) as 8 bytes each, v[t >> 1] dwords 2*(t & 1) (dims 0..3) and
 // 2*(t & 1) + 1 (dims 4..7). The A operand of block blk is byte blk of those
@@ -459,6 +480,11 @@ __device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T
   const bool prefix = P.tau_scope == SCHED_PD_TAU_PREFIX;
   const bool full = pos0 + 16u <= T.n && (T.budget == 0xFFFFFFFFu ||
                                           (prefix ? pos0 + 16u <= T.budget : so + 16u <= T.budget));
+  auto counts = [&](int v) __attribute__((always_inline)) {
+    const uint32_t i = 4u * g4 + v; // token in page (page size 16)
+    const uint32_t t = pos0 + i;
+    return t < T.n && (prefix ? t : so + i) < T.budget;
+  };
   float s[4];
 #pragma unroll
   for (int v = 0; v < 4; ++v)
@@ -466,9 +492,7 @@ __device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T
   if (!full) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const uint32_t i = 4u * g4 + v; // token in page (page size 16)
-      const uint32_t t = pos0 + i;
-      if (!(t < T.n && (prefix ? t : so + i) < T.budget))
+      if (!counts(v))
         s[v] = kNegInf;
     }
   }
@@ -541,6 +565,14 @@ __device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T
       vb[i] = B.v[i];
     if constexpr (!VT)
       bf16_v_operands(vb);
+    // Head dim 64 selects V of masked tokens to 0, as the VALU kernel does: a
+    // slot nobody wrote may hold a NaN, which p = 0 would not remove.
+    if constexpr (D == 64) {
+      if (!full) {
+        const bool in[4] = {counts(0), counts(1), counts(2), counts(3)};
+        mask_v64<VT>(vb, in);
+      }
+    }
   }
 #pragma unroll
   for (int blk = 0; blk < D / 16; ++blk) {
@@ -804,7 +836,7 @@ __device__ __forceinline__ void stream_urgent(const KParams &P, const MfmaTask &
 
 template <bool FP8, int NW, int GMAX, int DEPTH_S, int DEPTH_U, bool LINEAR = false,
           bool VT = false, bool PG = false, bool F16 = false, int D = 128, bool STOCK = false>
-__attribute__((amdgpu_waves_per_eu(STOCK ? 3 : 1)))
+__attribute__((amdgpu_waves_per_eu(STOCK || (D == 64 && PG) ? 3 : 1)))
 __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
   static_assert(!(F16 && (FP8 || LINEAR)), "fp16: softmax over an fp16 cache");
   static_assert(D == 128 || (D == 64 && !FP8 && !LINEAR), "head dim 64: softmax, 16-bit cache");

@@ -11,6 +11,7 @@ import torch
 import oracle
 import sched_pd
 import workloads
+from sched_rt import SchedPlane
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +42,44 @@ def test_d64_matches_the_oracle(kv, layout, ps, G):
     assert np.isnan(got[-1]).all()                  # an empty context: 0/0
     err = np.linalg.norm(got[:-1] - ref[:-1], axis=-1) / np.linalg.norm(ref[:-1], axis=-1)
     assert err.max() <= 4e-6, err.max()
+
+
+@pytest.mark.parametrize("kv", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout", ["tokmajor", "dmajor"])
+@pytest.mark.parametrize("ps", [16, 64])
+@pytest.mark.parametrize("shed", [False, True])
+def test_d64_reads_nothing_from_masked_slots(kv, layout, ps, shed):
+    """A pool the caller never cleared: NaN and infinities past every context
+    (and past every shed budget, whose pages are loaded and masked) leave the
+    output of a zeroed one, bit for bit."""
+    hkv, G = 2, 4
+    b = workloads.make_batch(np.asarray(CTX), num_q_heads=G * hkv, num_kv_heads=hkv, head_dim=64,
+                             page_size=ps, kv_dtype=kv, q_dtype=kv, seed=ps, device="cuda")
+    ctx = np.asarray(CTX)
+    seen = np.maximum(1, ctx // 2 + 1) if shed else ctx
+    kw = {}
+    if shed:
+        plane = SchedPlane(max_tasks=ctx.size * hkv)
+        plane.set_rows(tau=np.repeat(seen, hkv), n=ctx.size * hkv)
+        plane.push()
+        kw["plane"] = plane
+    live = torch.zeros(b["k_pool"].shape[0], ps, dtype=torch.bool, device="cuda")
+    bt = b["block_table"].cpu().numpy()
+    for r, n in enumerate(np.minimum(ctx, seen)):
+        for p in range(-(-int(n) // ps)):
+            live[int(bt[r, p]), :min(ps, int(n) - p * ps)] = True
+    outs = []
+    for bad in (0.0, float("nan"), float("inf")):
+        k = torch.where(live[:, None, :, None], b["k_pool"], bad)
+        v = torch.where(live[:, None, None, :], b["v_pool"], bad)
+        if layout == "tokmajor":
+            v = v.permute(0, 1, 3, 2).contiguous()
+        out = torch.full((len(CTX), G * hkv, 64), 7.0, device="cuda")
+        args = sched_pd.build_args(b["q"], k, v, b["block_table"], b["ctx_lens"], out=out,
+                                   v_layout=layout, **kw)
+        assert sched_pd.kernel_kind(args) == "mfma"
+        sched_pd.launch(args)
+        torch.cuda.synchronize()
+        outs.append(out[:-1].cpu())              # the last context is empty: 0/0
+    assert outs[0].isfinite().all()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
