@@ -515,21 +515,19 @@ __device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T
   // leave ~1.2e-3 relative error in the output (p is close to 1 for nearly
   // flat scores), so bf16 / fp8 carry p as hi + lo bf16 halves through two
   // MFMAs (~16 bits, the linear mode's split). fp16's 11 bits (~3e-4) are
-  // kept single. Head dim 64 carries p in full: three bf16 parts (24 bits),
-  // or fp16 hi + lo (22 bits, an absolute 2^-25 below that), so that its
-  // results stay those of an fp32 p; its pages have half the dim blocks to
-  // multiply, and the matrix cores are mostly idle either way.
-  u32x2_t pk, pl, p3;
-  if constexpr (F16) {
+  // kept single. Head dim 64 carries p in full, so that its results stay those
+  // of an fp32 p: in three bf16 parts (24 bits), or, over fp16 V, as fp32
+  // through the fp32 MFMAs: fp16 parts would stop at 2^-25, where a peaked row's
+  // tail lies (4093 tokens at p = 2^-26: 4e-3 off in hi + lo, 3.2e-5 here, 3.6e-5
+  // on the VALU kernel; 48 requests of 200..2900 tokens, fp16: 33.1 -> 38.5 us,
+  // VALU 163). Its pages have half the dim blocks to multiply, and the matrix
+  // cores are mostly idle either way.
+  u32x2_t pk = {0u, 0u}, pl, p3;
+  if constexpr (F16 && D == 64) {
+    // p stays fp32
+  } else if constexpr (F16) {
     pk.x = pack_f16_rne(p[0], p[1]);
     pk.y = pack_f16_rne(p[2], p[3]);
-    if constexpr (D == 64) {
-      // through scalars: a bit_cast of a vector's element reads element 0
-      const unsigned w0 = pk.x, w1 = pk.y;
-      const f16x2_t h0 = __builtin_bit_cast(f16x2_t, w0), h1 = __builtin_bit_cast(f16x2_t, w1);
-      pl.x = pack_f16_rne(p[0] - (float)h0.x, p[1] - (float)h0.y);
-      pl.y = pack_f16_rne(p[2] - (float)h1.x, p[3] - (float)h1.y);
-    }
   } else {
     float pv[4];
 #pragma unroll
@@ -586,9 +584,17 @@ __device__ __forceinline__ void compute_page(const KParams &P, const MfmaTask &T
                                                 : u32x2_t{vb[blk >> 1].x, vb[blk >> 1].y});
     else
       a = __builtin_bit_cast(s16x4_t, fp8x4_to_bf16x4(v8[blk]));
+    if constexpr (F16 && D == 64) {
+      // the lane's token 4*g4 + t is the operands' k index g4 of step t
+      const f16x4_t ah = __builtin_bit_cast(f16x4_t, a);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        S.acc[blk] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)ah[t], p[t], S.acc[blk], 0, 0, 0);
+      continue;
+    }
     S.acc[blk] = mfma_pv<F16>(a, pop, S.acc[blk]);
-    if constexpr (!F16 || D == 64)
-      S.acc[blk] = mfma_pv<F16>(a, __builtin_bit_cast(s16x4_t, pl), S.acc[blk]);
+    if constexpr (!F16)
+      S.acc[blk] = mfma_pv<false>(a, __builtin_bit_cast(s16x4_t, pl), S.acc[blk]);
     if constexpr (!F16 && D == 64)
       S.acc[blk] = mfma_pv<false>(a, __builtin_bit_cast(s16x4_t, p3), S.acc[blk]);
   }

@@ -2,8 +2,8 @@
 and of several 16-token blocks, groups at the edges of its q-head blocks,
 context lengths around page, block and wave boundaries. The fp32 output
 carries no rounding of its own, so the bound is the arithmetic's: p in full
-(24 bits in bf16 parts, 22 in fp16 ones) and fp32 sums of up to 3000 terms,
-a few 1e-7 of the row."""
+(24 bits in bf16 parts, fp32 over an fp16 cache) and fp32 sums of up to 3000
+terms, a few 1e-7 of the row."""
 import numpy as np
 import pytest
 import torch
@@ -83,3 +83,33 @@ def test_d64_reads_nothing_from_masked_slots(kv, layout, ps, shed):
         outs.append(out[:-1].cpu())              # the last context is empty: 0/0
     assert outs[0].isfinite().all()
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("kv", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout", ["tokmajor", "dmajor"])
+def test_d64_keeps_the_tail_of_a_peaked_row(kv, layout):
+    """A token in each of the first four pages (one for each wave of a task)
+    scores 18 above 4093 others, whose p = e^-18 = 2^-26 is far below a 16-bit
+    float's smallest step and whose V is 256 times larger: an output that drops
+    them is 0.4% off."""
+    n, ps = 4097, 16
+    b = workloads.make_batch(np.asarray([n]), num_q_heads=4, num_kv_heads=1, head_dim=64,
+                             page_size=ps, kv_dtype=kv, q_dtype=kv, seed=3, device="cuda")
+    q, k = torch.zeros_like(b["q"]), torch.zeros_like(b["k_pool"])
+    v = torch.full_like(b["v_pool"], 256.0)
+    first = b["block_table"][0, :4].long()
+    q[..., 0] = 12.0                             # 12 * 12 / sqrt(64) = 18
+    k[first, 0, 0, 0] = 12.0
+    v[first, 0, :, 0] = 1.0
+    if layout == "tokmajor":
+        v = v.permute(0, 1, 3, 2).contiguous()
+    out = torch.empty(1, 4, 64, device="cuda")
+    args = sched_pd.build_args(q, k, v, b["block_table"], b["ctx_lens"], out=out, v_layout=layout)
+    assert sched_pd.kernel_kind(args) == "mfma"
+    sched_pd.launch(args)
+    p = np.exp(-18.0)
+    want = (4.0 + 4093 * p * 256.0) / (4.0 + 4093 * p)
+    # a wave's fp32 sum adds 1024 tokens, fp32 MFMAs one at a time, and each add
+    # of this input may round by 2^-24 the same way: 6.1e-5
+    err = (out.double() / want - 1.0).abs().max().item()
+    assert err <= 6.1e-5
