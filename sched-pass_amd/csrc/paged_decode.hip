@@ -172,6 +172,9 @@ bool mfma_applies(const SchedDecodeArgs *a) {
     // token rows start 16-byte (16-bit V) or 8-byte (fp8 V) aligned
     if ((a->v_tok_stride * eb) % (a->kv_dtype == SCHED_PD_FP8_E4M3 ? 8 : 16))
       return false;
+    // a lane's offset in a block (12 rows and its dims at most) is 32 bits
+    if (a->v_tok_stride < 0 || a->v_tok_stride > (int64_t)((UINT32_MAX - 256u) / 12u) / eb)
+      return false;
   } else if (a->v_tok_stride != 1 || a->v_dim_stride != (int64_t)ps) {
     return false;
   }

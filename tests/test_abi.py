@@ -169,6 +169,22 @@ def test_kernel_selection(schedlib):
     assert kind(schedlib, fake_args(num_q_heads=16, num_kv_heads=8)) == 1  # d-major V: MFMA
 
 
+@pytest.mark.parametrize("d,kv,G", [(64, abi.BF16, 4), (64, abi.F16, 16), (128, abi.BF16, 4),
+                                    (128, abi.FP8_E4M3, 7)])
+def test_token_strides_past_a_lanes_32_bit_offset_leave_the_matrix_cores(schedlib, d, kv, G):
+    """The MFMA kernel's lanes reach the token rows 4 * (lane / 16) of a
+    token-major V block by a 32-bit offset: strides whose twelfth row lies past
+    it, and negative ones, go to the kernel with 64-bit offsets."""
+    eb = 1 if kv == abi.FP8_E4M3 else 2
+    q = abi.F16 if kv == abi.F16 else abi.BF16
+    base = dict(num_q_heads=G, num_kv_heads=1, head_dim=d, kv_dtype=kv, q_dtype=q, k_tok_stride=d,
+                v_dim_stride=1)
+    last = ((1 << 32) - 512) // 12 // eb // 16 * 16
+    for stride, want in ((d, 1), (last, 1), (last + 64, 0), (1 << 28, 0), (1 << 40, 0), (-d, 0)):
+        assert kind(schedlib, fake_args(**dict(base, v_tok_stride=stride))) == want, stride
+
+
+
 def prefetch_range(lib, a):
     lo, hi = ctypes.c_uint32(), ctypes.c_uint32()
     rc = lib.sched_paged_decode_prefetch_range(ctypes.byref(a), ctypes.byref(lo), ctypes.byref(hi))
