@@ -412,8 +412,10 @@ def build_args(q, k_pool, v_pool, block_table, ctx_lens, *, out,
 def _split_on_device(a, block_table, page_indptr, device, stream) -> None:
     """Let the library cut the tasks of a launch without tiles into work items
     (sched_paged_decode_auto_split), with a workspace of the launch stream. A
-    launch that is being captured gets one of its own, cleared in the graph:
-    graphs captured on one stream may be replayed on several."""
+    launch that is being captured gets one of its own, cleared in the graph
+    (graphs captured on one stream may be replayed on several), from the memory
+    pool that lives as long as the graph; a capture without such a pool (a raw
+    stream capture, not torch.cuda.graph) runs whole tasks, which need none."""
     if page_indptr is None:
         longest, mean = block_table.shape[1], 0
     else:
@@ -425,6 +427,10 @@ def _split_on_device(a, block_table, page_indptr, device, stream) -> None:
     counters = WS_COUNTERS_OFF + 4 * a.num_requests * a.num_kv_heads
     if torch.cuda.is_current_stream_capturing():
         ws = torch.empty(need, dtype=torch.uint8, device=device)
+        if not _in_private_pool(ws):
+            a.flags &= ~abi.FLAG_SPLIT
+            a.num_tiles = a.tile_pages = 0
+            return
         ws[:counters].zero_()
     else:
         # one per (thread, stream): between a thread's clear and its launch no
@@ -434,6 +440,14 @@ def _split_on_device(a, block_table, page_indptr, device, stream) -> None:
             cache = _SPLIT_WS.streams = {}
         ws = workspace_for(need, device, stream=stream, count_bytes=counters, _cache=cache)
     a.workspace, a.workspace_bytes, a._ws = ws.data_ptr(), ws.numel(), ws
+
+
+def _in_private_pool(t) -> bool:
+    """Whether the caching allocator took `t` from a graph's (or MemPool's) own
+    pool; memory of the ordinary pool goes to other tensors once `t` is dropped."""
+    p = t.data_ptr()
+    return any(s["address"] <= p < s["address"] + s["total_size"]
+               and tuple(s["segment_pool_id"]) != (0, 0) for s in torch.cuda.memory_snapshot())
 
 
 _WS = {}

@@ -164,6 +164,38 @@ def test_csr_table_and_graph_replays(schedlib):
         assert torch.equal(run(pos, kw).nan_to_num(9.0), base)
 
 
+def test_raw_stream_capture_holds_no_freed_memory(schedlib):
+    """A capture that torch does not manage keeps no pool for what is allocated
+    under it: such a launch is captured whole, with no workspace (one node, the
+    decode's), and its replays leave tensors allocated later alone."""
+    import ctypes
+    hip = ctypes.CDLL("libamdhip64.so")
+    pos, kw, hkv, tol = make("bf16")
+    base = run(pos, kw).nan_to_num(9.0)
+    out = torch.empty_like(base)
+    side = torch.cuda.Stream()
+    graph, exe, nodes = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_size_t()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        h = ctypes.c_void_p(side.cuda_stream)
+        assert hip.hipStreamBeginCapture(h, 1) == 0         # thread-local mode
+        sched_pd.paged_decode(*pos, out=out, **kw)
+        assert hip.hipStreamEndCapture(h, ctypes.byref(graph)) == 0
+        assert hip.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0
+        assert nodes.value == 1
+        assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None,
+                                       ctypes.c_size_t(0)) == 0
+        fillers = [torch.full((1 << 18,), 3, dtype=torch.uint8, device="cuda") for _ in range(64)]
+        for _ in range(3):
+            out.fill_(7.0)
+            assert hip.hipGraphLaunch(exe, h) == 0
+            side.synchronize()
+            got = out.nan_to_num(9.0)
+            assert ((got - base).norm(dim=-1) <= 2 * tol * base.norm(dim=-1)).all()
+        assert all((f == 3).all().item() for f in fillers)
+        assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph) == 0
+
+
 def test_threads_on_one_stream(schedlib):
     """Launches of several threads' shapes interleave on the default stream: each
     thread's workspace keeps its counters."""
