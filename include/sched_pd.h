@@ -338,8 +338,10 @@ int64_t sched_paged_decode_workspace_bytes(const SchedDecodeArgs *a);
  * on the device, and if so set SCHED_PD_FLAG_SPLIT, tile_pages and num_tiles
  * in *a. max_pages bounds a request's pages; mean_pages is their mean over the
  * requests, 0 if the caller does not know it. pi, num_tasks, order_size and the
- * queue still count tasks. Returns the workspace bytes the launch then needs (0:
- * not split, -1: invalid arguments). No counterpart in the reference. */
+ * queue still count tasks. The three are cleared first, so one block may be
+ * decided again for another shape (a block with tiles keeps tile_pages and
+ * num_tiles). Returns the workspace bytes the launch then needs (0: not split,
+ * -1: invalid arguments). No counterpart in the reference. */
 int64_t sched_paged_decode_auto_split(SchedDecodeArgs *a, uint32_t max_pages,
                                       uint32_t mean_pages);
 

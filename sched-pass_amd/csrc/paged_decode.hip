@@ -779,7 +779,12 @@ int64_t sched_paged_decode_auto_split(SchedDecodeArgs *a, uint32_t max_pages,
                                       uint32_t mean_pages) {
   KParams kp;
   Selected sel;
-  if (a == nullptr || prepare(a, &kp, &sel))
+  if (a == nullptr)
+    return -1;
+  a->flags &= ~SCHED_PD_FLAG_SPLIT; // what an earlier call decided is not this shape's
+  if (a->tiles == nullptr)
+    a->tile_pages = a->num_tiles = 0;
+  if (prepare(a, &kp, &sel))
     return -1;
   const uint64_t ntasks = kp.ntasks;
   if (a->tiles || ntasks == 0 || max_pages == 0)

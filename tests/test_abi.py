@@ -611,3 +611,26 @@ def test_graded_plan_rows_by_position_in_the_claim_order():
             sched_pd.plan_graded_host(ctx, 16, 1, sizes=bad)
     with pytest.raises(ValueError):
         sched_pd.plan_graded_host(ctx, 16, 1, task_order=[0, 0, 1])
+
+
+def test_auto_split_decides_a_refilled_block_afresh(schedlib):
+    """One argument block per step: what an earlier call set is not left behind
+    when the next shape is whole, or has another number of tasks, and a block
+    with tiles keeps its plan."""
+    def split(a, pages):
+        return schedlib.sched_paged_decode_auto_split(ctypes.byref(a), pages, 0)
+    a = fake_args(num_requests=1)
+    need = split(a, 512)
+    assert need > 0 and a.flags & abi.FLAG_SPLIT and a.num_tiles >= 16 and a.tile_pages
+    assert split(a, 1) == 0                                  # too short to split
+    assert not a.flags & abi.FLAG_SPLIT and a.num_tiles == a.tile_pages == 0
+    assert kind(schedlib, a) == 1                            # launches, with no workspace
+    assert split(a, 512) == need
+    a.num_requests = 3                                       # num_tiles no multiple of 24
+    assert split(a, 512) > need
+    a.num_q_heads = 31                                       # refused: nothing left either
+    assert split(a, 512) == -1
+    assert not a.flags & abi.FLAG_SPLIT and a.num_tiles == a.tile_pages == 0
+    t = fake_args(tiles=ctypes.c_void_p(0x90000), num_tiles=8, tile_pages=4,
+                  workspace=ctypes.c_void_p(0xA0000), workspace_bytes=1 << 20)
+    assert split(t, 512) == 0 and (t.num_tiles, t.tile_pages) == (8, 4)
