@@ -345,9 +345,10 @@ int64_t sched_paged_decode_workspace_bytes(const SchedDecodeArgs *a);
 int64_t sched_paged_decode_auto_split(SchedDecodeArgs *a, uint32_t max_pages,
                                       uint32_t mean_pages);
 
-/* Work items resident per CU for the kernel `a` selects (workgroups per CU,
- * times the tasks a workgroup of the one-wave-per-task kernel runs; 0 =
- * unknown). Counterpart of reference paged_softmax_occupancy
+/* Work items resident per CU for the kernel that `a` selects with lever tables,
+ * whether it names any yet or not (workgroups per CU, times the tasks a workgroup
+ * of the one-wave-per-task kernel runs; 0 = unknown): the W a queue launch is
+ * sized by. Counterpart of reference paged_softmax_occupancy
  * (python/kernels/paged_softmax.cu:61-67), whose CTAs are tasks. */
 int sched_paged_decode_occupancy(const SchedDecodeArgs *a);
 

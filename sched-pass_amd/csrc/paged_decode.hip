@@ -260,8 +260,9 @@ bool stock_launch(const SchedDecodeArgs *a, const KParams &kp) {
          (a->mode == SCHED_PD_LINEAR || (kts >= 0 && kts <= (INT32_MAX - 64) / 16));
 }
 
-// Validate `a`; on success fill *kp (tables resolved) and *sel.
-int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel) {
+// Validate `a`; on success fill *kp (tables resolved) and *sel (`levers`: the
+// kernel a launch with lever tables runs, though `a` names none).
+int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = false) {
   if (a == nullptr)
     return set_error(hipErrorInvalidValue, "args is NULL");
   if (a->abi_version != SCHED_PD_ABI_VERSION)
@@ -428,7 +429,7 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel) {
     sel->per_block = SCHED_PD_WAVE_NWT;
   } else if (mfma) {
     const bool pg = a->page_size > 16;
-    const bool stock = stock_launch(a, *kp), vt = v_token_major(a);
+    const bool stock = !levers && stock_launch(a, *kp), vt = v_token_major(a);
     if (a->head_dim == 64)
       sel->fn = a->kv_dtype == SCHED_PD_F16 ? mfma_kernel_d64<true>(G, vt, pg, stock)
                                             : mfma_kernel_d64<false>(G, vt, pg, stock);
@@ -823,9 +824,11 @@ int64_t sched_paged_decode_auto_split(SchedDecodeArgs *a, uint32_t max_pages,
 }
 
 int sched_paged_decode_occupancy(const SchedDecodeArgs *a) {
+  // asked, often before any table is there, to size a queue or an order: the
+  // lever kernel's (the lever-free form of the same shape holds 3 to its 2)
   KParams kp;
   Selected sel;
-  if (prepare(a, &kp, &sel))
+  if (prepare(a, &kp, &sel, true))
     return 0;
   int blocks = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, sel.fn, sel.block, 0) != hipSuccess)

@@ -57,3 +57,20 @@ def test_stock_and_lever_forms_agree(schedlib, kv, q, layout, ps, form):
                                        **kw), np.float64)
         err = np.abs(outs[0].double().numpy() - ref).max(-1) / np.abs(ref).max(-1)
         assert err.max() <= 2 ** -8, err.max()
+
+
+@pytest.mark.parametrize("kv,q,d", [(torch.bfloat16, torch.bfloat16, 128),
+                                    (torch.float16, torch.float16, 64),
+                                    (torch.float8_e4m3fn, torch.bfloat16, 128),
+                                    (torch.float32, torch.float32, 64)])
+def test_occupancy_is_the_lever_forms_before_any_table_is_armed(schedlib, kv, q, d):
+    """A queue's worker count is asked of arguments that name no tables yet."""
+    b = workloads.make_batch(np.asarray(CTX), num_q_heads=8, num_kv_heads=2, head_dim=d,
+                             page_size=16, kv_dtype=kv, q_dtype=q, seed=1, device="cuda")
+    got = []
+    for plane in (None, SchedPlane(max_tasks=len(CTX) * 2)):
+        out = torch.empty(len(CTX), 8, d, device="cuda")
+        got.append(sched_pd.occupancy(sched_pd.build_args(
+            b["q"], b["k_pool"], b["v_pool"], b["block_table"], b["ctx_lens"], out=out,
+            plane=plane, k_scale=b.get("k_scale"), v_scale=b.get("v_scale"))))
+    assert got[0] == got[1] > 0
