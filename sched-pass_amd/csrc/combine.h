@@ -229,7 +229,7 @@ __device__ __forceinline__ void finish_item(const KParams &P, uint32_t wi, uint3
   __syncthreads();
   __shared__ uint32_t s_last;
   if (threadIdx.x == 0)
-    s_last = (P.L.nsub > 1u ? arrive_chunk(P.ws_count + task, chunk, nchunks)
+    s_last = (P.sub.nsub > 1u ? arrive_chunk(P.ws_count + task, chunk, nchunks)
                             : arrive(P.ws_count + task, nchunks))
                  ? 1u
                  : 0u;
@@ -244,8 +244,8 @@ __device__ __forceinline__ void finish_item(const KParams &P, uint32_t wi, uint3
 // following from the context length. Ranged rows (task, chunk | nchunks << 16,
 // p0, p1) carry the task's chunk count and the chunk's page range, so the
 // chunks of one task may differ in size. Without a list, work item = task, or
-// (L.nsub > 1) item task * nsub + chunk: the task's pages in up to `nsub` equal
-// chunks of split_pages or more, so few or ragged tasks spread over the chip
+// (sub.nsub > 1) item task * nsub + chunk: the task's pages in up to `nsub` equal
+// chunks of sub.pages or more, so few or ragged tasks spread over the chip
 // with no plan (one request of 8191 tokens, 32 / 8 heads: 73 -> 17 us). The
 // chunk size follows from the context alone, never from a shed budget or the
 // schedule, so the levers leave every bit as it is here too.
@@ -253,11 +253,12 @@ struct ItemRow {
   uint32_t task, chunk, nchunks, p0, p1;
 };
 
+template <bool SPLIT = true>
 __device__ __forceinline__ ItemRow item_row(const KParams &P, uint32_t wi) {
   ItemRow I{wi, 0u, 1u, 0u, 0u};
-  if (__builtin_expect(P.L.nsub > 1u, 0)) {
-    I.task = wi / P.L.nsub;
-    I.chunk = wi - I.task * P.L.nsub;
+  if (__builtin_expect(sub_items<SPLIT>(P.sub) > 1u, 0)) {
+    I.task = wi / P.sub.nsub;
+    I.chunk = wi - I.task * P.sub.nsub;
     return I;
   }
   if (P.tiles == nullptr)
@@ -281,16 +282,17 @@ __device__ __forceinline__ ItemRow item_row(const KParams &P, uint32_t wi) {
 // the npages_load pages of the task that are read at all (n context tokens).
 struct ItemRange {
   uint32_t nchunks, p0, p1;
-  uint32_t cp; // L.nsub > 1: pages per chunk
+  uint32_t cp; // sub.nsub > 1: pages per chunk
 };
 
+template <bool SPLIT = true>
 __device__ __forceinline__ ItemRange item_range(const KParams &P, const ItemRow &I, uint32_t n,
                                                 uint32_t npages_load) {
-  if (__builtin_expect(P.L.nsub > 1u, 0)) {
+  if (__builtin_expect(sub_items<SPLIT>(P.sub) > 1u, 0)) {
     // chunks wholly past a budget are skipped (the merge of a masked chunk
     // would add exact zeros)
     ItemRange it;
-    it.cp = max(P.split_pages, ((n + P.ps - 1u) / P.ps + P.L.nsub - 1u) / P.L.nsub);
+    it.cp = max(P.sub.pages, ((n + P.ps - 1u) / P.ps + P.sub.nsub - 1u) / P.sub.nsub);
     it.nchunks = max(1u, (npages_load + it.cp - 1u) / it.cp);
     it.p0 = min(I.chunk * it.cp, npages_load);
     it.p1 = min(it.p0 + it.cp, npages_load);
@@ -329,9 +331,10 @@ __device__ __forceinline__ ItemRange item_range(const KParams &P, const ItemRow 
 // partial. Every item of a task reads the same rows and lengths, so they all
 // decide alike. The merge only ever reads items [wi - chunk, wi - chunk +
 // nchunks), which a running item keeps inside the list.
+template <bool SPLIT = true>
 __device__ __forceinline__ bool item_skip(const KParams &P, uint32_t wi, const ItemRow &I,
                                          const ItemRange &R) {
-  return (P.L.nsub > 1u && I.chunk >= R.nchunks) ||
+  return (sub_items<SPLIT>(P.sub) > 1u && I.chunk >= R.nchunks) ||
          (P.tiles != nullptr && (I.chunk > wi || I.chunk >= R.nchunks));
 }
 

@@ -37,7 +37,6 @@ struct KParams {
   uint32_t ntasks;     // requests x kv-heads
   uint32_t tile_pages;
   uint32_t tile_ranged; // rows (task, chunk | nchunks << 16, p0, p1), else (task, chunk)
-  uint32_t split_pages; // L.nsub > 1: fewest pages of a task's item (SCHED_PD_FLAG_SPLIT)
   uint32_t *ws_stale;  // tasks found with a stale plan (item_stale)
   uint32_t *ws_count;  // per-task arrival counters
   float *ws_ml;        // per-work-item (m, l) per head
@@ -50,6 +49,7 @@ struct KParams {
   uint32_t app_f32;       // fp32 source rows (else the cache's 16-bit type, or for an fp8
                           // cache app_f16 ? fp16 : bf16)
   uint32_t app_f16;
+  SubItems sub;
 };
 
 constexpr float kNegInf = -__builtin_huge_valf();

@@ -857,7 +857,7 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
   const bool toff = STOCK || timer_off_latched(P.L);
   constexpr uint32_t EB = FP8 ? 1u : 2u; // bytes per KV element
 
-  run_tasks(P.L, [&](uint32_t wi, bool last_round) __attribute__((always_inline)) {
+  run_tasks(P.L, P.sub, [&](uint32_t wi, bool last_round) __attribute__((always_inline)) {
     if (wi >= P.L.nitems)
       return;
     const unsigned long long t0 = STOCK ? 0ull : read_clock(P.L.wallclock);
@@ -904,7 +904,7 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
       if (P.app_k != nullptr && T.n > 0u) {
         const uint32_t pos = T.n - 1u, pg = pos / P.ps;
         const bool holds =
-            P.L.nsub > 1u ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
+            P.sub.nsub > 1u ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
             P.tiles == nullptr ||
             (P.tile_ranged ? pg >= I.p0 && pg < I.p1 : I.chunk == pg / P.tile_pages);
         if (holds || (stale && I.chunk == 0u)) {

@@ -159,8 +159,9 @@ template <typename KVT, int D> struct WaveChunk {
 // NWT + wave, remapped by pi over the launch's items) or the ticket queue
 // (W worker waves; claim after the body, lane 0's atomic, broadcast by
 // readfirstlane). Same decisions as run_tasks, per wave.
-template <int NWT, class Body>
-__device__ __forceinline__ void run_wave_tasks(const LeverTables &L, Body &&body) {
+template <int NWT, bool SPLIT, class Body>
+__device__ __forceinline__ void run_wave_tasks(const LeverTables &L, const SubItems &S,
+                                               Body &&body) {
   const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t pid = blockIdx.x * NWT + w;
   uint32_t ntasks = 0u;
@@ -186,13 +187,13 @@ __device__ __forceinline__ void run_wave_tasks(const LeverTables &L, Body &&body
     }
     for (uint32_t v = v0; v < L.nitems; v += gridDim.x * NWT) {
       uint32_t chunk;
-      const uint32_t pos = sub_position(L, v, false, &chunk);
-      body(remap_static(L, pos, L.npi) * L.nsub + chunk);
+      const uint32_t pos = sub_position<SPLIT>(S, v, false, &chunk);
+      body(remap_static(L, pos, SPLIT ? S.npi : L.nitems) * sub_items<SPLIT>(S) + chunk);
     }
     return;
   }
   const uint32_t W = L.workers, npos = ntasks;
-  ntasks *= L.nsub;
+  ntasks *= sub_items<SPLIT>(S);
   if (pid >= W || pid >= ntasks)
     return;
   const uint32_t last_ticket = W + ntasks - 1u;
@@ -200,8 +201,8 @@ __device__ __forceinline__ void run_wave_tasks(const LeverTables &L, Body &&body
   uint32_t raw = pid;
   while (true) {
     uint32_t chunk;
-    const uint32_t pos = sub_position(L, raw, true, &chunk);
-    body(remap_wq(L, pos, npos) * L.nsub + chunk);
+    const uint32_t pos = sub_position<SPLIT>(S, raw, true, &chunk);
+    body(remap_wq(L, pos, npos) * sub_items<SPLIT>(S) + chunk);
     uint32_t t = 0u;
     if (lane == 0u) {
       t = __hip_atomic_fetch_add(lt_queue(L), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -222,7 +223,7 @@ __device__ __forceinline__ void run_wave_tasks(const LeverTables &L, Body &&body
 // its partial's stores before its arrival atomic; the reading item loads
 // only after its own arrival has returned (see the handoff note at the top
 // of combine.h).
-template <int G, int VN, int D>
+template <int G, int VN, int D, bool SPLIT>
 __device__ __forceinline__ void finish_wave_item(const KParams &P, uint32_t wi, uint32_t task,
                                                  uint32_t chunk, uint32_t nchunks, uint32_t r,
                                                  uint32_t h, const WaveState<VN> (&st)[G],
@@ -258,7 +259,7 @@ __device__ __forceinline__ void finish_wave_item(const KParams &P, uint32_t wi, 
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   uint32_t last = 0u;
   if (lane == 0u)
-    last = (P.L.nsub > 1u ? arrive_chunk(P.ws_count + task, chunk, nchunks)
+    last = (sub_items<SPLIT>(P.sub) > 1u ? arrive_chunk(P.ws_count + task, chunk, nchunks)
                           : arrive(P.ws_count + task, nchunks))
                ? 1u
                : 0u;
@@ -266,7 +267,11 @@ __device__ __forceinline__ void finish_wave_item(const KParams &P, uint32_t wi, 
     merge_partials<D, float, false>(P, wi - chunk, nchunks, G, orow, lane, 64u);
 }
 
-template <typename KVT, int D, int NWT, int G>
+// SPLIT: launches with sub-items (SCHED_PD_FLAG_SPLIT) run a form of their own.
+// In one form for both, the sub-item arithmetic costs the small launches, whose
+// start is most of their time: 200 requests through launch_paged_softmax 8.53 ->
+// 8.88 us, 1267 requests 11.2 -> 11.5.
+template <typename KVT, int D, int NWT, int G, bool SPLIT>
 __global__ void __launch_bounds__(NWT * 64) decode_wave(KParams P) {
   using S = WaveShape<KVT, D>;
   constexpr int VN = S::VN, LPR = S::LPR, TPI = S::TPI, NI = S::NI, DEPTH = S::DEPTH;
@@ -275,11 +280,11 @@ __global__ void __launch_bounds__(NWT * 64) decode_wave(KParams P) {
   const uint32_t ts = lane / LPR, ds = lane % LPR;
   const bool toff = timer_off_latched(P.L);
 
-  run_wave_tasks<NWT>(P.L, [&](uint32_t wi) __attribute__((always_inline)) {
+  run_wave_tasks<NWT, SPLIT>(P.L, P.sub, [&](uint32_t wi) __attribute__((always_inline)) {
     if (wi >= P.L.nitems)
       return;
     const unsigned long long t0 = read_clock(P.L.wallclock);
-    const ItemRow I = item_row(P, wi);
+    const ItemRow I = item_row<SPLIT>(P, wi);
     const uint32_t task = I.task;
     if (task >= P.ntasks)
       return;
@@ -288,8 +293,8 @@ __global__ void __launch_bounds__(NWT * 64) decode_wave(KParams P) {
     const uint32_t n = ctx_tokens(P, r);
     const uint32_t nload = load_extent(P, n, pol.budget);
     const uint32_t ps = P.ps, cpp = ps / 16u; // 16-token chunks per page
-    const ItemRange R = item_range(P, I, n, (nload + ps - 1u) / ps);
-    if (item_skip(P, wi, I, R))
+    const ItemRange R = item_range<SPLIT>(P, I, n, (nload + ps - 1u) / ps);
+    if (item_skip<SPLIT>(P, wi, I, R))
       return;
     const bool stale = item_stale(P, wi, I, R, n);
     // the item's 16-token chunks [c_begin, c_end) of those read
@@ -305,7 +310,7 @@ __global__ void __launch_bounds__(NWT * 64) decode_wave(KParams P) {
       if (P.app_k != nullptr && n > 0u) {
         const uint32_t pos = n - 1u, pg = pos / ps;
         const bool holds =
-            P.L.nsub > 1u ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
+            sub_items<SPLIT>(P.sub) > 1u ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
             P.tiles == nullptr ||
             (P.tile_ranged ? pg >= I.p0 && pg < I.p1 : I.chunk == pg / P.tile_pages);
         if (holds || (stale && I.chunk == 0u)) {
@@ -520,7 +525,7 @@ __global__ void __launch_bounds__(NWT * 64) decode_wave(KParams P) {
           __hip_atomic_fetch_add(P.ws_stale, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     } else {
-      finish_wave_item<G, VN, D>(P, wi, task, I.chunk, R.nchunks, r, h, st, lane, ts, ds);
+      finish_wave_item<G, VN, D, SPLIT>(P, wi, task, I.chunk, R.nchunks, r, h, st, lane, ts, ds);
     }
     unsigned long long *timer = lt_timer(P.L);
     if (lane == 0u && timer != nullptr && task < P.L.max_tasks && !toff) {

@@ -162,7 +162,9 @@ constexpr int mfma_du(bool fp8, bool vt, bool pg, bool f16 = false) {
 // One wave per work item (softmax, token-major rows), G = 1..3 q-heads per
 // kv-head: one group per translation unit.
 #define SCHED_PD_WAVE_ONE(PRE, KVT, D, G)                                                        \
-  PRE template __global__ void schedpd::decode_wave<KVT, D, SCHED_PD_WAVE_NWT, G>(               \
+  PRE template __global__ void schedpd::decode_wave<KVT, D, SCHED_PD_WAVE_NWT, G, false>(        \
+      schedpd::KParams);                                                                         \
+  PRE template __global__ void schedpd::decode_wave<KVT, D, SCHED_PD_WAVE_NWT, G, true>(         \
       schedpd::KParams);
 #define SCHED_PD_WAVE_G(PRE, G)                                                                  \
   SCHED_PD_WAVE_ONE(PRE, float, 32, G)                                                           \

@@ -21,9 +21,6 @@ struct LeverTables {
   uint32_t *queue;           // ticket counter
   uint32_t max_tasks;        // rows in order/ctrl/timer
   uint32_t nitems;           // work items of this launch (static grid size)
-  uint32_t npi;              // positions of pi on the static grid (nitems / nsub)
-  uint32_t nsub;             // items of each position of pi and of the queue (1, or a split
-                             // task's: SCHED_PD_FLAG_SPLIT)
   uint32_t wq;               // 1 = launched as W persistent workers
   uint32_t workers;          // W of a work-queue launch (per-wave kernels)
   uint32_t spread;           // per-wave kernels, static grid: workgroups resident at once
@@ -36,6 +33,16 @@ struct LeverTables {
   // takes effect at the next launch.
   uint64_t rt_slot[4];
   uint32_t rt;
+};
+
+// A launch whose tasks are split on the device (SCHED_PD_FLAG_SPLIT; else nsub
+// = 1). Last in the kernel's arguments: among the tables it changed the loads
+// that every launch starts with (200 requests through launch_paged_softmax: 8.53
+// -> 8.59 us; the queue over 256 ragged requests: 357.9 -> 359.5).
+struct SubItems {
+  uint32_t nsub;  // items of each position of pi and of the queue
+  uint32_t npi;   // positions of pi on the static grid (nitems / nsub)
+  uint32_t pages; // fewest pages of an item
 };
 
 struct TaskPolicy {
@@ -117,23 +124,28 @@ __device__ __forceinline__ uint32_t remap_wq(const LeverTables &L, uint32_t raw,
   return ok ? mapped : raw;
 }
 
-// With sub-items (L.nsub > 1) pi, num_tasks and the queue's positions are
+// With sub-items (nsub > 1) pi, num_tasks and the queue's positions are
 // tasks: the task position of grid position or ticket `raw`, and which of its
 // items. On a static grid the first item of every task comes first, so those
 // past a context's end (which only look at its length) come last; a task's
-// items take consecutive tickets.
-__device__ __forceinline__ uint32_t sub_position(const LeverTables &L, uint32_t raw, bool queue,
+// items take consecutive tickets. Here and in combine.h, SPLIT = false is a
+// kernel whose launches have no sub-items (nsub == 1, known on the host).
+template <bool SPLIT> __device__ __forceinline__ uint32_t sub_items(const SubItems &S) {
+  return SPLIT ? S.nsub : 1u;
+}
+template <bool SPLIT = true>
+__device__ __forceinline__ uint32_t sub_position(const SubItems &S, uint32_t raw, bool queue,
                                                  uint32_t *chunk) {
   *chunk = 0u;
-  if (__builtin_expect(L.nsub <= 1u, 1))
+  if (__builtin_expect(sub_items<SPLIT>(S) <= 1u, 1))
     return raw;
   if (queue) {
-    const uint32_t pos = raw / L.nsub;
-    *chunk = raw - pos * L.nsub;
+    const uint32_t pos = raw / S.nsub;
+    *chunk = raw - pos * S.nsub;
     return pos;
   }
-  *chunk = raw / L.npi;
-  return raw - *chunk * L.npi;
+  *chunk = raw / S.npi;
+  return raw - *chunk * S.npi;
 }
 
 // Policy flags and shed budget of one task (reference lib/SchedWeave.cpp:
@@ -207,13 +219,13 @@ __device__ __forceinline__ void timer_commit(const LeverTables &L, bool off, uin
 // item per workgroup.
 template <bool V> struct NoLevers {};
 template <class Body, bool STOCK = false>
-__device__ __forceinline__ void run_tasks(const LeverTables &L, Body &&body,
+__device__ __forceinline__ void run_tasks(const LeverTables &L, const SubItems &S, Body &&body,
                                           NoLevers<STOCK> = NoLevers<STOCK>()) {
   const uint32_t pid = blockIdx.x;
   uint32_t chunk;
   if constexpr (STOCK) {
-    const uint32_t pos = sub_position(L, pid, false, &chunk);
-    body(__builtin_amdgcn_readfirstlane(pos * L.nsub + chunk), false);
+    const uint32_t pos = sub_position(S, pid, false, &chunk);
+    body(__builtin_amdgcn_readfirstlane(pos * S.nsub + chunk), false);
     return;
   }
   uint32_t ntasks = 0u;
@@ -224,7 +236,7 @@ __device__ __forceinline__ void run_tasks(const LeverTables &L, Body &&body,
   }
   const bool queue = ntasks != 0u;
   const uint32_t npos = ntasks; // what pi and num_tasks count
-  ntasks *= L.nsub;
+  ntasks *= S.nsub;
   if (queue && pid >= ntasks)
     return;
   __shared__ uint32_t s_next;
@@ -247,10 +259,10 @@ __device__ __forceinline__ void run_tasks(const LeverTables &L, Body &&body,
     // with fewer and fewer others beside it
     const bool last_round = queue && ntasks >= 2u * gridDim.x &&
                             raw + SCHED_PD_LATE_ROUNDS * gridDim.x >= ntasks;
-    const uint32_t pos = sub_position(L, raw, queue, &chunk);
+    const uint32_t pos = sub_position(S, raw, queue, &chunk);
     const uint32_t item =
-        queue ? remap_wq(L, pos, npos) : remap_static(L, pos, L.npi);
-    body(__builtin_amdgcn_readfirstlane(item * L.nsub + chunk),
+        queue ? remap_wq(L, pos, npos) : remap_static(L, pos, S.npi);
+    body(__builtin_amdgcn_readfirstlane(item * S.nsub + chunk),
          last_round);
     if (!queue) {
       raw += gridDim.x;

@@ -233,22 +233,24 @@ bool wave_applies(const SchedDecodeArgs *a) {
   return aligned16(a->k_pool) && aligned16(a->v_pool);
 }
 
-template <int G> KernelFn wave_kernel_g(const SchedDecodeArgs *a) {
+template <int G, bool SPLIT> KernelFn wave_kernel_g(const SchedDecodeArgs *a) {
   constexpr int NWT = SCHED_PD_WAVE_NWT;
   if (a->kv_dtype == SCHED_PD_F32)
-    return a->head_dim == 32   ? decode_wave<float, 32, NWT, G>
-           : a->head_dim == 64 ? decode_wave<float, 64, NWT, G>
-                               : decode_wave<float, 128, NWT, G>;
+    return a->head_dim == 32   ? decode_wave<float, 32, NWT, G, SPLIT>
+           : a->head_dim == 64 ? decode_wave<float, 64, NWT, G, SPLIT>
+                               : decode_wave<float, 128, NWT, G, SPLIT>;
   if (a->kv_dtype == SCHED_PD_BF16)
-    return a->head_dim == 64 ? decode_wave<uint16_t, 64, NWT, G>
-                             : decode_wave<uint16_t, 128, NWT, G>;
-  return a->head_dim == 64 ? decode_wave<_Float16, 64, NWT, G>
-                           : decode_wave<_Float16, 128, NWT, G>;
+    return a->head_dim == 64 ? decode_wave<uint16_t, 64, NWT, G, SPLIT>
+                             : decode_wave<uint16_t, 128, NWT, G, SPLIT>;
+  return a->head_dim == 64 ? decode_wave<_Float16, 64, NWT, G, SPLIT>
+                           : decode_wave<_Float16, 128, NWT, G, SPLIT>;
 }
 
-KernelFn wave_kernel(const SchedDecodeArgs *a) {
+template <bool SPLIT> KernelFn wave_kernel(const SchedDecodeArgs *a) {
   const uint32_t G = a->num_q_heads / a->num_kv_heads;
-  return G == 1 ? wave_kernel_g<1>(a) : G == 2 ? wave_kernel_g<2>(a) : wave_kernel_g<3>(a);
+  return G == 1   ? wave_kernel_g<1, SPLIT>(a)
+         : G == 2 ? wave_kernel_g<2, SPLIT>(a)
+                  : wave_kernel_g<3, SPLIT>(a);
 }
 
 // A launch with no lever tables at all (no pi, control block, timer, queue or
@@ -345,8 +347,8 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = 
   }
   kp->ntasks = a->num_requests * a->num_kv_heads;
   kp->L.nitems = kp->ntasks;
-  kp->L.nsub = 1u;
-  kp->L.npi = kp->ntasks;
+  kp->sub.nsub = 1u;
+  kp->sub.npi = kp->ntasks;
   const bool split = a->tiles == nullptr && (a->flags & SCHED_PD_FLAG_SPLIT);
   if (split) {
     if (kp->ntasks == 0 || a->tile_pages == 0 || a->num_tiles < 2u * kp->ntasks ||
@@ -354,8 +356,8 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = 
       return set_error(hipErrorInvalidValue,
                        "split tasks need tile_pages > 0 and num_tiles a multiple (2 to 32) of "
                        "the %u tasks", kp->ntasks);
-    kp->L.nsub = a->num_tiles / kp->ntasks;
-    kp->split_pages = a->tile_pages;
+    kp->sub.nsub = a->num_tiles / kp->ntasks;
+    kp->sub.pages = a->tile_pages;
   }
   if (a->tiles || split) {
     if (a->tiles && a->tile_format > SCHED_PD_TILES_RANGED)
@@ -374,7 +376,7 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = 
     kp->tile_pages = a->tile_pages;
     kp->tile_ranged = a->tile_format == SCHED_PD_TILES_RANGED ? 1u : 0u;
     kp->L.nitems = a->num_tiles;
-    kp->L.npi = a->num_tiles / kp->L.nsub;
+    kp->sub.npi = a->num_tiles / kp->sub.nsub;
     kp->ws_stale = reinterpret_cast<uint32_t *>(ws + W.stale_off);
     kp->ws_count = reinterpret_cast<uint32_t *>(ws + W.count_off);
     kp->ws_ml = reinterpret_cast<float *>(ws + W.ml_off);
@@ -423,7 +425,7 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = 
 
   sel->per_block = 1;
   if (wave) {
-    sel->fn = wave_kernel(a);
+    sel->fn = split ? wave_kernel<true>(a) : wave_kernel<false>(a);
     sel->block = SCHED_PD_WAVE_NWT * 64;
     sel->mfma = 2;
     sel->per_block = SCHED_PD_WAVE_NWT;
@@ -672,7 +674,7 @@ static int launch_decode(const SchedDecodeArgs *a, const AppendRows *app, void *
   hipError_t e = hipGetLastError();
   if (e != hipSuccess)
     return set_error(e, "kernel launch failed: %s", hipGetErrorString(e));
-  if (kp.L.nsub > 1u && (kp.L.order != nullptr || kp.L.rt)) {
+  if (kp.sub.nsub > 1u && (kp.L.order != nullptr || kp.L.rt)) {
     // pi may have named a task twice, whose second run's arrivals stay: the
     // next launch on this workspace starts from clear words again
     launch_zero_words(kp.ws_count, kp.ntasks, stream);
