@@ -982,7 +982,7 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
       __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
     if constexpr (STOCK) {
       if (T.p1 - T.p0 > kLongItemPages)
-        stream_pages<FP8, NW, DEPTH_S, false, LINEAR, VT, PG, F16, D, true>(P, T, S, lane, g4);
+        stream_pages<FP8, NW, DEPTH_U, false, LINEAR, VT, PG, F16, D, true>(P, T, S, lane, g4);
       else
         stream_pages<FP8, NW, DEPTH_S, kStockNT, LINEAR, VT, PG, F16, D, true>(P, T, S, lane, g4);
     } else if ((T.p1 - T.p0 > kLongItemPages || (kLateDeep && last_round)) && !pol.polite)

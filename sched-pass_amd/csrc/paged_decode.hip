@@ -58,9 +58,9 @@ template <typename KVT, int D> KernelFn valu_kernel(bool linear, uint32_t G) {
 template <bool FP8, bool VT = false, bool PG = false>
 KernelFn mfma_kernel(uint32_t G, bool linear, bool stock) {
   constexpr int NW = SCHED_PD_MFMA_NW, DS = mfma_ds(FP8), DU = mfma_du(FP8, VT, PG),
-                D0 = mfma_stock(FP8, VT);
+                D0 = mfma_stock(FP8, VT), DL = mfma_stock_du(FP8, VT, PG, true);
   if (linear)
-    return stock ? decode_mfma<FP8, NW, 4, D0, D0, true, VT, PG, false, 128, true>
+    return stock ? decode_mfma<FP8, NW, 4, D0, DL, true, VT, PG, false, 128, true>
                  : decode_mfma<FP8, NW, 4, DS, DU, true, VT, PG, false>;
   if (stock)
     return G <= 4   ? decode_mfma<FP8, NW, 4, D0, D0, false, VT, PG, false, 128, true>
