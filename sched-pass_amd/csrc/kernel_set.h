@@ -52,8 +52,9 @@
 #define SCHED_PD_MFMA_DEPTH_D64 4
 #endif
 
-// The launches without lever tables (decode_mfma's STOCK): fp8 token-major V
-// at depth 4 spills within the 168 registers of three waves per SIMD; 3 fits.
+// The launches without lever tables (decode_mfma's STOCK): fp8 token-major V of
+// 16-token pages at depth 4 spills within the 168 registers of three waves per
+// SIMD; 3 fits. (Larger pages and the linear mode hold 4: 158 and 147.)
 #ifndef SCHED_PD_MFMA_DEPTH_FP8_VT_STOCK
 #define SCHED_PD_MFMA_DEPTH_FP8_VT_STOCK 3
 #endif
@@ -61,9 +62,8 @@
 namespace schedpd {
 
 constexpr int mfma_ds(bool fp8) { return fp8 ? SCHED_PD_MFMA_DEPTH_FP8 : SCHED_PD_MFMA_DEPTH; }
-constexpr int mfma_stock(bool fp8, bool vt) {
-  return fp8 ? (vt ? SCHED_PD_MFMA_DEPTH_FP8_VT_STOCK : SCHED_PD_MFMA_DEPTH_FP8)
-             : SCHED_PD_MFMA_DEPTH;
+constexpr int mfma_stock(bool fp8, bool vt, bool pg, bool linear) {
+  return fp8 && vt && !pg && !linear ? SCHED_PD_MFMA_DEPTH_FP8_VT_STOCK : mfma_ds(fp8);
 }
 // Deepest ring (the urgent default). An urgent task's ring depth is any of
 // mfma_ds .. mfma_du (SchedDecodeArgs.pf_dist).
@@ -80,7 +80,7 @@ constexpr int mfma_du(bool fp8, bool vt, bool pg, bool f16 = false) {
 // tokens, 8 heads, bf16: 74.6 -> 49.3 us, the lever form 50.6); the softmax forms'
 // does not fit three waves' registers.
 constexpr int mfma_stock_du(bool fp8, bool vt, bool pg, bool linear) {
-  return linear ? mfma_du(fp8, vt, pg) : mfma_stock(fp8, vt);
+  return linear ? mfma_du(fp8, vt, pg) : mfma_stock(fp8, vt, pg, linear);
 }
 
 } // namespace schedpd
@@ -93,7 +93,7 @@ constexpr int mfma_stock_du(bool fp8, bool vt, bool pg, bool linear) {
                                                     schedpd::mfma_du(FP8, VT, PG, F16), LIN, VT, PG, F16>( \
       schedpd::KParams);                                                                         \
   PRE template __global__ void schedpd::decode_mfma<FP8, SCHED_PD_MFMA_NW, GMAX,                 \
-                                                    schedpd::mfma_stock(FP8, VT),                \
+                                                    schedpd::mfma_stock(FP8, VT, PG, LIN),       \
                                                     schedpd::mfma_stock_du(FP8, VT, PG, LIN),    \
                                                     LIN, VT, PG, F16, 128, true>(schedpd::KParams);
 #define SCHED_PD_MFMA_SOFTMAX(PRE, FP8, VT, PG, F16)                                             \

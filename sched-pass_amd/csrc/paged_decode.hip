@@ -58,9 +58,9 @@ template <typename KVT, int D> KernelFn valu_kernel(bool linear, uint32_t G) {
 template <bool FP8, bool VT = false, bool PG = false>
 KernelFn mfma_kernel(uint32_t G, bool linear, bool stock) {
   constexpr int NW = SCHED_PD_MFMA_NW, DS = mfma_ds(FP8), DU = mfma_du(FP8, VT, PG),
-                D0 = mfma_stock(FP8, VT), DL = mfma_stock_du(FP8, VT, PG, true);
+                D0 = mfma_stock(FP8, VT, PG, false), DL = mfma_stock_du(FP8, VT, PG, true);
   if (linear)
-    return stock ? decode_mfma<FP8, NW, 4, D0, DL, true, VT, PG, false, 128, true>
+    return stock ? decode_mfma<FP8, NW, 4, DS, DL, true, VT, PG, false, 128, true>
                  : decode_mfma<FP8, NW, 4, DS, DU, true, VT, PG, false>;
   if (stock)
     return G <= 4   ? decode_mfma<FP8, NW, 4, D0, D0, false, VT, PG, false, 128, true>
@@ -78,7 +78,7 @@ uint32_t elem_bytes(uint32_t dt) {
 // fp16 cache with fp16 Q: 16-byte page-16 layouts, softmax mode.
 template <bool VT, bool PG = false> KernelFn mfma_kernel_f16(uint32_t G, bool stock) {
   constexpr int NW = SCHED_PD_MFMA_NW, DS = mfma_ds(false), DU = mfma_du(false, VT, PG, true),
-                D0 = mfma_stock(false, VT);
+                D0 = mfma_stock(false, VT, PG, false);
   if (stock)
     return G <= 4   ? decode_mfma<false, NW, 4, D0, D0, false, VT, PG, true, 128, true>
            : G <= 8 ? decode_mfma<false, NW, 8, D0, D0, false, VT, PG, true, 128, true>
@@ -262,6 +262,25 @@ bool stock_launch(const SchedDecodeArgs *a, const KParams &kp) {
          (a->mode == SCHED_PD_LINEAR || (kts >= 0 && kts <= (INT32_MAX - 64) / 16));
 }
 
+// fp8 token-major V of 16-token pages, softmax: the lever-free form's ring of 3
+// pages and its K exchange make a lone item's stream 5 to 11% slower than the
+// lever form's ring of 4 (one request of 2001 tokens, 8 kv-heads: 22.9 -> 24.6 us;
+// 232 items over 128-page tiles: 26.6 -> 28.3), which its third workgroup per CU
+// outweighs only once there are items for two (336 items of 2001 tokens: 43.4 ->
+// 36.8; 488 of up to 128 pages: 52.4 -> 45.0). Short items gain from the shorter
+// start (480 of 201 tokens: 12.1 -> 9.0; 8 of 201: 8.7 -> 6.5). So launches of at
+// most a workgroup per CU whose items may be long keep the lever form.
+constexpr uint32_t kLoneItems = 256, kLoneItemPages = 64;
+
+bool lone_fp8_items(const SchedDecodeArgs *a, const KParams &kp) {
+  if (a->kv_dtype != SCHED_PD_FP8_E4M3 || a->mode == SCHED_PD_LINEAR || !v_token_major(a) ||
+      a->page_size != 16 || kp.L.nitems > kLoneItems)
+    return false;
+  if (a->tiles != nullptr)
+    return kp.tile_ranged || a->tile_pages > kLoneItemPages;
+  return kp.sub.nsub > 1u || a->page_indptr != nullptr || a->bt_stride > kLoneItemPages;
+}
+
 // Validate `a`; on success fill *kp (tables resolved) and *sel (`levers`: the
 // kernel a launch with lever tables runs, though `a` names none).
 int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = false) {
@@ -431,7 +450,8 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = 
     sel->per_block = SCHED_PD_WAVE_NWT;
   } else if (mfma) {
     const bool pg = a->page_size > 16;
-    const bool stock = !levers && stock_launch(a, *kp), vt = v_token_major(a);
+    const bool stock = !levers && stock_launch(a, *kp) && !lone_fp8_items(a, *kp);
+    const bool vt = v_token_major(a);
     if (a->head_dim == 64)
       sel->fn = a->kv_dtype == SCHED_PD_F16 ? mfma_kernel_d64<true>(G, vt, pg, stock)
                                             : mfma_kernel_d64<false>(G, vt, pg, stock);

@@ -59,6 +59,30 @@ def test_stock_and_lever_forms_agree(schedlib, kv, q, layout, ps, form):
         assert err.max() <= 2 ** -8, err.max()
 
 
+@pytest.mark.parametrize("ctx", [CTX * 10, [c for c in CTX if c <= 1024], [1024] * 3, [1025] * 3])
+def test_fp8_token_major_forms_agree(schedlib, ctx):
+    """fp8 token-major V of 16-token pages runs the lever-free form once there
+    are more than 256 items, or none longer than 64 pages: on both sides of both
+    lines the lever form's bits and the oracle's values."""
+    b = workloads.make_batch(np.asarray(ctx), num_q_heads=10, num_kv_heads=2, head_dim=128,
+                             page_size=16, kv_dtype=torch.float8_e4m3fn, q_dtype=torch.bfloat16,
+                             seed=7, device="cuda")
+    v = b["v_pool"].permute(0, 1, 3, 2).contiguous()
+    kw = dict(v_layout="tokmajor", k_scale=b.get("k_scale"), v_scale=b.get("v_scale"))
+    outs = []
+    for plane in (None, SchedPlane(max_tasks=len(ctx) * 2)):
+        out = torch.full((len(ctx), 10, 128), 7.0, device="cuda")
+        sched_pd.launch(sched_pd.build_args(b["q"], b["k_pool"], v, b["block_table"],
+                                            b["ctx_lens"], out=out, plane=plane, **kw))
+        torch.cuda.synchronize()
+        outs.append(out.cpu())
+    assert torch.equal(outs[0], outs[1])
+    ref = np.asarray(oracle.decode(b["q"], b["k_pool"], v, b["block_table"], b["ctx_lens"], **kw),
+                     np.float64)
+    err = np.abs(outs[0].double().numpy() - ref).max(-1) / np.abs(ref).max(-1)
+    assert err.max() <= 2 ** -8, err.max()
+
+
 @pytest.mark.parametrize("kv,q,d", [(torch.bfloat16, torch.bfloat16, 128),
                                     (torch.float16, torch.float16, 64),
                                     (torch.float8_e4m3fn, torch.bfloat16, 128),
