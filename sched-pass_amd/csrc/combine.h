@@ -229,7 +229,7 @@ __device__ __forceinline__ void finish_item(const KParams &P, uint32_t wi, uint3
   __syncthreads();
   __shared__ uint32_t s_last;
   if (threadIdx.x == 0)
-    s_last = (P.sub.nsub > 1u ? arrive_chunk(P.ws_count + task, chunk, nchunks)
+    s_last = (sub_items<true>(P.L) > 1u ? arrive_chunk(P.ws_count + task, chunk, nchunks)
                             : arrive(P.ws_count + task, nchunks))
                  ? 1u
                  : 0u;
@@ -244,7 +244,7 @@ __device__ __forceinline__ void finish_item(const KParams &P, uint32_t wi, uint3
 // following from the context length. Ranged rows (task, chunk | nchunks << 16,
 // p0, p1) carry the task's chunk count and the chunk's page range, so the
 // chunks of one task may differ in size. Without a list, work item = task, or
-// (sub.nsub > 1) item task * nsub + chunk: the task's pages in up to `nsub` equal
+// (nsub > 1) item task * nsub + chunk: the task's pages in up to `nsub` equal
 // chunks of sub.pages or more, so few or ragged tasks spread over the chip
 // with no plan (one request of 8191 tokens, 32 / 8 heads: 73 -> 17 us). The
 // chunk size follows from the context alone, never from a shed budget or the
@@ -256,9 +256,9 @@ struct ItemRow {
 template <bool SPLIT = true>
 __device__ __forceinline__ ItemRow item_row(const KParams &P, uint32_t wi) {
   ItemRow I{wi, 0u, 1u, 0u, 0u};
-  if (__builtin_expect(sub_items<SPLIT>(P.sub) > 1u, 0)) {
-    I.task = wi / P.sub.nsub;
-    I.chunk = wi - I.task * P.sub.nsub;
+  if (__builtin_expect(sub_items<SPLIT>(P.L) > 1u, 0)) {
+    I.task = wi / sub_items<SPLIT>(P.L);
+    I.chunk = wi - I.task * sub_items<SPLIT>(P.L);
     return I;
   }
   if (P.tiles == nullptr)
@@ -282,17 +282,18 @@ __device__ __forceinline__ ItemRow item_row(const KParams &P, uint32_t wi) {
 // the npages_load pages of the task that are read at all (n context tokens).
 struct ItemRange {
   uint32_t nchunks, p0, p1;
-  uint32_t cp; // sub.nsub > 1: pages per chunk
+  uint32_t cp; // nsub > 1: pages per chunk
 };
 
 template <bool SPLIT = true>
 __device__ __forceinline__ ItemRange item_range(const KParams &P, const ItemRow &I, uint32_t n,
                                                 uint32_t npages_load) {
-  if (__builtin_expect(sub_items<SPLIT>(P.sub) > 1u, 0)) {
+  if (__builtin_expect(sub_items<SPLIT>(P.L) > 1u, 0)) {
     // chunks wholly past a budget are skipped (the merge of a masked chunk
     // would add exact zeros)
     ItemRange it;
-    it.cp = max(P.sub.pages, ((n + P.ps - 1u) / P.ps + P.sub.nsub - 1u) / P.sub.nsub);
+    const uint32_t nsub = sub_items<SPLIT>(P.L);
+    it.cp = max(P.sub.pages, ((n + P.ps - 1u) / P.ps + nsub - 1u) / nsub);
     it.nchunks = max(1u, (npages_load + it.cp - 1u) / it.cp);
     it.p0 = min(I.chunk * it.cp, npages_load);
     it.p1 = min(it.p0 + it.cp, npages_load);
@@ -334,7 +335,7 @@ __device__ __forceinline__ ItemRange item_range(const KParams &P, const ItemRow 
 template <bool SPLIT = true>
 __device__ __forceinline__ bool item_skip(const KParams &P, uint32_t wi, const ItemRow &I,
                                          const ItemRange &R) {
-  return (sub_items<SPLIT>(P.sub) > 1u && I.chunk >= R.nchunks) ||
+  return (sub_items<SPLIT>(P.L) > 1u && I.chunk >= R.nchunks) ||
          (P.tiles != nullptr && (I.chunk > wi || I.chunk >= R.nchunks));
 }
 

@@ -842,7 +842,7 @@ __device__ __forceinline__ void stream_urgent(const KParams &P, const MfmaTask &
 
 template <bool FP8, int NW, int GMAX, int DEPTH_S, int DEPTH_U, bool LINEAR = false,
           bool VT = false, bool PG = false, bool F16 = false, int D = 128, bool STOCK = false>
-__attribute__((amdgpu_waves_per_eu(STOCK || (D == 64 && PG) ? 3 : 1)))
+__attribute__((amdgpu_waves_per_eu(STOCK || (D == 64 && PG && (VT || !F16)) ? 3 : 1)))
 __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
   static_assert(!(F16 && (FP8 || LINEAR)), "fp16: softmax over an fp16 cache");
   static_assert(D == 128 || (D == 64 && !FP8 && !LINEAR), "head dim 64: softmax, 16-bit cache");
@@ -904,7 +904,7 @@ __global__ void __launch_bounds__(NW * 64) decode_mfma(KParams P) {
       if (P.app_k != nullptr && T.n > 0u) {
         const uint32_t pos = T.n - 1u, pg = pos / P.ps;
         const bool holds =
-            P.sub.nsub > 1u ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
+            sub_items<true>(P.L) > 1u ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
             P.tiles == nullptr ||
             (P.tile_ranged ? pg >= I.p0 && pg < I.p1 : I.chunk == pg / P.tile_pages);
         if (holds || (stale && I.chunk == 0u)) {

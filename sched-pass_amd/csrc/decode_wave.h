@@ -165,7 +165,7 @@ __device__ __forceinline__ void run_wave_tasks(const LeverTables &L, const SubIt
   const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t pid = blockIdx.x * NWT + w;
   uint32_t ntasks = 0u;
-  if (L.wq) {
+  if (L.wq & 1u) {
     const bool armed = lt_queue(L) != nullptr && lt_ctrl(L) != nullptr && gridDim.y == 1 &&
                        gridDim.z == 1;
     ntasks = armed ? ld_u32(lt_ctrl(L) + SCHED_CTRL_NUM_TASKS_OFF) : 0u;
@@ -187,13 +187,13 @@ __device__ __forceinline__ void run_wave_tasks(const LeverTables &L, const SubIt
     }
     for (uint32_t v = v0; v < L.nitems; v += gridDim.x * NWT) {
       uint32_t chunk;
-      const uint32_t pos = sub_position<SPLIT>(S, v, false, &chunk);
-      body(remap_static(L, pos, SPLIT ? S.npi : L.nitems) * sub_items<SPLIT>(S) + chunk);
+      const uint32_t pos = sub_position<SPLIT>(L, S, v, false, &chunk);
+      body(remap_static(L, pos, SPLIT ? S.npi : L.nitems) * sub_items<SPLIT>(L) + chunk);
     }
     return;
   }
   const uint32_t W = L.workers, npos = ntasks;
-  ntasks *= sub_items<SPLIT>(S);
+  ntasks *= sub_items<SPLIT>(L);
   if (pid >= W || pid >= ntasks)
     return;
   const uint32_t last_ticket = W + ntasks - 1u;
@@ -201,8 +201,8 @@ __device__ __forceinline__ void run_wave_tasks(const LeverTables &L, const SubIt
   uint32_t raw = pid;
   while (true) {
     uint32_t chunk;
-    const uint32_t pos = sub_position<SPLIT>(S, raw, true, &chunk);
-    body(remap_wq(L, pos, npos) * sub_items<SPLIT>(S) + chunk);
+    const uint32_t pos = sub_position<SPLIT>(L, S, raw, true, &chunk);
+    body(remap_wq(L, pos, npos) * sub_items<SPLIT>(L) + chunk);
     uint32_t t = 0u;
     if (lane == 0u) {
       t = __hip_atomic_fetch_add(lt_queue(L), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -259,7 +259,7 @@ __device__ __forceinline__ void finish_wave_item(const KParams &P, uint32_t wi, 
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   uint32_t last = 0u;
   if (lane == 0u)
-    last = (sub_items<SPLIT>(P.sub) > 1u ? arrive_chunk(P.ws_count + task, chunk, nchunks)
+    last = (sub_items<SPLIT>(P.L) > 1u ? arrive_chunk(P.ws_count + task, chunk, nchunks)
                           : arrive(P.ws_count + task, nchunks))
                ? 1u
                : 0u;
@@ -310,7 +310,7 @@ __global__ void __launch_bounds__(NWT * 64) decode_wave(KParams P) {
       if (P.app_k != nullptr && n > 0u) {
         const uint32_t pos = n - 1u, pg = pos / ps;
         const bool holds =
-            sub_items<SPLIT>(P.sub) > 1u ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
+            sub_items<SPLIT>(P.L) > 1u ? I.chunk == min(pg / R.cp, R.nchunks - 1u) :
             P.tiles == nullptr ||
             (P.tile_ranged ? pg >= I.p0 && pg < I.p1 : I.chunk == pg / P.tile_pages);
         if (holds || (stale && I.chunk == 0u)) {

@@ -21,7 +21,9 @@ struct LeverTables {
   uint32_t *queue;           // ticket counter
   uint32_t max_tasks;        // rows in order/ctrl/timer
   uint32_t nitems;           // work items of this launch (static grid size)
-  uint32_t wq;               // 1 = launched as W persistent workers
+  uint32_t wq;               // bit 0: launched as W persistent workers; bits 8 and up: items
+                             // of each position of pi and of the queue (1, or those of a
+                             // task split on the device, SCHED_PD_FLAG_SPLIT)
   uint32_t workers;          // W of a work-queue launch (per-wave kernels)
   uint32_t spread;           // per-wave kernels, static grid: workgroups resident at once
                              // (0 or 1: positions row-major, wave-minor)
@@ -35,12 +37,12 @@ struct LeverTables {
   uint32_t rt;
 };
 
-// A launch whose tasks are split on the device (SCHED_PD_FLAG_SPLIT; else nsub
-// = 1). Last in the kernel's arguments: among the tables it changed the loads
-// that every launch starts with (200 requests through launch_paged_softmax: 8.53
-// -> 8.59 us; the queue over 256 ragged requests: 357.9 -> 359.5).
+// A launch whose tasks are split on the device, read only there. Last in the
+// kernel's arguments, and the item count in wq's word, so that the loads every
+// launch starts with are those of a launch without it. Fields among the tables
+// cost 0.1 us on 200 requests through launch_paged_softmax (8.53 -> 8.67), a count
+// at the arguments' end 0.4 us on 72 items of an fp8 step (28.6 -> 29.0).
 struct SubItems {
-  uint32_t nsub;  // items of each position of pi and of the queue
   uint32_t npi;   // positions of pi on the static grid (nitems / nsub)
   uint32_t pages; // fewest pages of an item
 };
@@ -130,18 +132,19 @@ __device__ __forceinline__ uint32_t remap_wq(const LeverTables &L, uint32_t raw,
 // past a context's end (which only look at its length) come last; a task's
 // items take consecutive tickets. Here and in combine.h, SPLIT = false is a
 // kernel whose launches have no sub-items (nsub == 1, known on the host).
-template <bool SPLIT> __device__ __forceinline__ uint32_t sub_items(const SubItems &S) {
-  return SPLIT ? S.nsub : 1u;
+template <bool SPLIT> __host__ __device__ __forceinline__ uint32_t sub_items(const LeverTables &L) {
+  return SPLIT ? L.wq >> 8 : 1u;
 }
 template <bool SPLIT = true>
-__device__ __forceinline__ uint32_t sub_position(const SubItems &S, uint32_t raw, bool queue,
-                                                 uint32_t *chunk) {
+__device__ __forceinline__ uint32_t sub_position(const LeverTables &L, const SubItems &S,
+                                                 uint32_t raw, bool queue, uint32_t *chunk) {
   *chunk = 0u;
-  if (__builtin_expect(sub_items<SPLIT>(S) <= 1u, 1))
+  const uint32_t nsub = sub_items<SPLIT>(L);
+  if (__builtin_expect(nsub <= 1u, 1))
     return raw;
   if (queue) {
-    const uint32_t pos = raw / S.nsub;
-    *chunk = raw - pos * S.nsub;
+    const uint32_t pos = raw / nsub;
+    *chunk = raw - pos * nsub;
     return pos;
   }
   *chunk = raw / S.npi;
@@ -224,19 +227,20 @@ __device__ __forceinline__ void run_tasks(const LeverTables &L, const SubItems &
   const uint32_t pid = blockIdx.x;
   uint32_t chunk;
   if constexpr (STOCK) {
-    const uint32_t pos = sub_position(S, pid, false, &chunk);
-    body(__builtin_amdgcn_readfirstlane(pos * S.nsub + chunk), false);
+    const uint32_t pos = sub_position(L, S, pid, false, &chunk);
+    body(__builtin_amdgcn_readfirstlane(pos * sub_items<true>(L) + chunk), false);
     return;
   }
   uint32_t ntasks = 0u;
-  if (L.wq) {
+  if (L.wq & 1u) {
     const bool grid1d = gridDim.y == 1 && gridDim.z == 1;
     const bool armed = lt_queue(L) != nullptr && lt_ctrl(L) != nullptr && grid1d;
     ntasks = armed ? ld_u32(lt_ctrl(L) + SCHED_CTRL_NUM_TASKS_OFF) : 0u;
   }
   const bool queue = ntasks != 0u;
   const uint32_t npos = ntasks; // what pi and num_tasks count
-  ntasks *= S.nsub;
+  const uint32_t nsub = sub_items<true>(L);
+  ntasks *= nsub;
   if (queue && pid >= ntasks)
     return;
   __shared__ uint32_t s_next;
@@ -259,10 +263,10 @@ __device__ __forceinline__ void run_tasks(const LeverTables &L, const SubItems &
     // with fewer and fewer others beside it
     const bool last_round = queue && ntasks >= 2u * gridDim.x &&
                             raw + SCHED_PD_LATE_ROUNDS * gridDim.x >= ntasks;
-    const uint32_t pos = sub_position(S, raw, queue, &chunk);
+    const uint32_t pos = sub_position(L, S, raw, queue, &chunk);
     const uint32_t item =
-        queue ? remap_wq(L, pos, npos) : remap_static(L, pos, S.npi);
-    body(__builtin_amdgcn_readfirstlane(item * S.nsub + chunk),
+        queue ? remap_wq(L, pos, npos) : remap_static(L, pos, nsub > 1u ? S.npi : L.nitems);
+    body(__builtin_amdgcn_readfirstlane(item * nsub + chunk),
          last_round);
     if (!queue) {
       raw += gridDim.x;

@@ -278,7 +278,7 @@ bool lone_fp8_items(const SchedDecodeArgs *a, const KParams &kp) {
     return false;
   if (a->tiles != nullptr)
     return kp.tile_ranged || a->tile_pages > kLoneItemPages;
-  return kp.sub.nsub > 1u || a->page_indptr != nullptr || a->bt_stride > kLoneItemPages;
+  return sub_items<true>(kp.L) > 1u || a->page_indptr != nullptr || a->bt_stride > kLoneItemPages;
 }
 
 // Validate `a`; on success fill *kp (tables resolved) and *sel (`levers`: the
@@ -366,7 +366,7 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = 
   }
   kp->ntasks = a->num_requests * a->num_kv_heads;
   kp->L.nitems = kp->ntasks;
-  kp->sub.nsub = 1u;
+  uint32_t nsub = 1u;
   kp->sub.npi = kp->ntasks;
   const bool split = a->tiles == nullptr && (a->flags & SCHED_PD_FLAG_SPLIT);
   if (split) {
@@ -375,7 +375,7 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = 
       return set_error(hipErrorInvalidValue,
                        "split tasks need tile_pages > 0 and num_tiles a multiple (2 to 32) of "
                        "the %u tasks", kp->ntasks);
-    kp->sub.nsub = a->num_tiles / kp->ntasks;
+    nsub = a->num_tiles / kp->ntasks;
     kp->sub.pages = a->tile_pages;
   }
   if (a->tiles || split) {
@@ -395,12 +395,13 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = 
     kp->tile_pages = a->tile_pages;
     kp->tile_ranged = a->tile_format == SCHED_PD_TILES_RANGED ? 1u : 0u;
     kp->L.nitems = a->num_tiles;
-    kp->sub.npi = a->num_tiles / kp->sub.nsub;
+    kp->sub.npi = a->num_tiles / nsub;
     kp->ws_stale = reinterpret_cast<uint32_t *>(ws + W.stale_off);
     kp->ws_count = reinterpret_cast<uint32_t *>(ws + W.count_off);
     kp->ws_ml = reinterpret_cast<float *>(ws + W.ml_off);
     kp->ws_acc = ws + W.acc_off;
   }
+  kp->L.wq = nsub << 8;
   kp->L.wallclock = (a->flags & SCHED_PD_FLAG_WALLCLOCK) ? 1u : 0u;
   kp->L.dT = a->policy_dT;
   kp->L.dR = a->policy_dR;
@@ -686,7 +687,7 @@ static int launch_decode(const SchedDecodeArgs *a, const AppendRows *app, void *
   }
   const uint32_t slots = wq ? a->workers : nitems;
   const uint32_t grid = (slots + sel.per_block - 1) / sel.per_block;
-  kp.L.wq = wq ? 1u : 0u;
+  kp.L.wq |= wq ? 1u : 0u;
   kp.L.workers = wq ? a->workers : 0u;
   if (sel.per_block > 1 && !wq)
     kp.L.spread = min(grid, resident_blocks(reinterpret_cast<const void *>(sel.fn), sel.block));
@@ -694,7 +695,7 @@ static int launch_decode(const SchedDecodeArgs *a, const AppendRows *app, void *
   hipError_t e = hipGetLastError();
   if (e != hipSuccess)
     return set_error(e, "kernel launch failed: %s", hipGetErrorString(e));
-  if (kp.sub.nsub > 1u && (kp.L.order != nullptr || kp.L.rt)) {
+  if (sub_items<true>(kp.L) > 1u && (kp.L.order != nullptr || kp.L.rt)) {
     // pi may have named a task twice, whose second run's arrivals stay: the
     // next launch on this workspace starts from clear words again
     launch_zero_words(kp.ws_count, kp.ntasks, stream);
