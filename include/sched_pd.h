@@ -209,7 +209,8 @@ uint64_t sched_rt_timer_host_va(void);
                                            general VALU kernel */
 #define SCHED_PD_FLAG_SPLIT 0x80u       /* with tiles NULL: each task runs as up to num_tiles /
                                            (requests x kv-heads) work items of tile_pages
-                                           pages or more, cut from the context on the device
+                                           pages or more, cut from the context on the device;
+                                           a task little longer than one item is whole
                                            (sched_paged_decode_auto_split fills these in) */
 #define SCHED_PD_FLAG_NO_MFMA 0x40u     /* do not use the MFMA kernel: the one-wave-per-item
                                            kernel where it applies, else the VALU kernel */
@@ -336,8 +337,12 @@ int64_t sched_paged_decode_workspace_bytes(const SchedDecodeArgs *a);
 
 /* For a launch without tiles: decide from its shape whether its tasks are split
  * on the device, and if so set SCHED_PD_FLAG_SPLIT, tile_pages and num_tiles
- * in *a. max_pages bounds a request's pages; mean_pages is their mean over the
- * requests, 0 if the caller does not know it. pi, num_tasks, order_size and the
+ * in *a. max_pages bounds a request's pages (a loose bound only makes the grid
+ * larger); mean_pages is their mean over the requests, 0 if the caller does not
+ * know it. A task's chunks, and so the last bits of its output, follow from its
+ * context, the shape, the number of tasks and mean_pages: equal under every lever
+ * and table width, not across batches (a launch without the flag does not depend
+ * on the batch). pi, num_tasks, order_size and the
  * queue still count tasks. The three are cleared first, so one block may be
  * decided again for another shape (a block with tiles keeps tile_pages and
  * num_tiles). Returns the workspace bytes the launch then needs (0: not split,

@@ -44,7 +44,8 @@ struct LeverTables {
 // at the arguments' end 0.4 us on 72 items of an fp8 step (28.6 -> 29.0).
 struct SubItems {
   uint32_t npi;   // positions of pi on the static grid (nitems / nsub)
-  uint32_t pages; // fewest pages of an item
+  uint32_t pages; // pages that an item is worth
+  uint32_t from;  // pages from which a task is split
 };
 
 struct TaskPolicy {

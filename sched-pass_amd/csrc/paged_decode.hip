@@ -233,6 +233,20 @@ bool wave_applies(const SchedDecodeArgs *a) {
   return aligned16(a->k_pool) && aligned16(a->v_pool);
 }
 
+// The matrix cores wherever the MFMA kernel applies (a d-major V included:
+// the general VALU kernel reads it 3.7x slower); the one-wave kernel for
+// groups of 1-3 over token-major rows that the MFMA kernel does not take
+// (fp32 KV or Q, head dim 32 / 64); below kMfmaMinGroup the one-wave
+// kernel first unless the launch asks for an urgent prefetch depth
+// (pf_dist), which only the MFMA kernel's ring serves.
+bool mfma_allowed(const SchedDecodeArgs *a) {
+  return !(a->flags & SCHED_PD_FLAG_NO_MFMA) && mfma_applies(a);
+}
+bool wave_launch(const SchedDecodeArgs *a) {
+  const uint32_t G = a->mode == SCHED_PD_LINEAR ? 1u : a->num_q_heads / a->num_kv_heads;
+  return wave_applies(a) && (!mfma_allowed(a) || (G < kMfmaMinGroup && a->pf_dist == 0));
+}
+
 template <int G, bool SPLIT> KernelFn wave_kernel_g(const SchedDecodeArgs *a) {
   constexpr int NWT = SCHED_PD_WAVE_NWT;
   if (a->kv_dtype == SCHED_PD_F32)
@@ -281,6 +295,22 @@ bool lone_fp8_items(const SchedDecodeArgs *a, const KParams &kp) {
   return sub_items<true>(kp.L) > 1u || a->page_indptr != nullptr || a->bt_stride > kLoneItemPages;
 }
 
+// Task counts between which the split's rule changes (sched_paged_decode_auto_split).
+constexpr uint32_t kFewTasks = 128, kRoundTasks = 256, kFullTasks = 512, kOverTasks = 1024;
+
+// Pages from which a split launch splits a task, where an item is worth `least`:
+// 5/4 of it, but 5/2 where the tasks are a workgroup per CU or nearly, or two and
+// more, and tasks of one length keep every CU busy by themselves and in two items
+// only pay for the merge (192 fp8 tasks of 129 pages: 20.5 us whole, 25.8 in two;
+// 256 bf16 ones 43 and 47; 512 of mean 70, at most 383: 71 and 87); a page list's
+// mean keeps full launches whole by itself. The one-wave kernel's small items: twice
+// (8 fp32 tasks of 6 pages: 6.7 whole, 8.2 in two).
+uint64_t split_from(const SchedDecodeArgs *a, uint64_t ntasks, uint64_t least) {
+  const bool full = ntasks > kFewTasks && (ntasks <= kRoundTasks ||
+                                           (ntasks >= kFullTasks && a->page_indptr == nullptr));
+  return least * (wave_launch(a) ? 8u : full ? 10u : 5u) / 4u;
+}
+
 // Validate `a`; on success fill *kp (tables resolved) and *sel (`levers`: the
 // kernel a launch with lever tables runs, though `a` names none).
 int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = false) {
@@ -325,16 +355,8 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = 
     return set_error(hipErrorInvalidValue, "bt_stride is 0 with a 2-D block table");
 
   const int64_t eb = elem_bytes(a->kv_dtype);
-  // The matrix cores wherever the MFMA kernel applies (a d-major V included:
-  // the general VALU kernel reads it 3.7x slower); the one-wave kernel for
-  // groups of 1-3 over token-major rows that the MFMA kernel does not take
-  // (fp32 KV or Q, head dim 32 / 64); below kMfmaMinGroup the one-wave
-  // kernel first unless the launch asks for an urgent prefetch depth
-  // (pf_dist), which only the MFMA kernel's ring serves.
-  const bool mfma_ok = !(a->flags & SCHED_PD_FLAG_NO_MFMA) && mfma_applies(a);
-  const bool wave_ok = wave_applies(a);
-  const bool wave = wave_ok && (!mfma_ok || (G < kMfmaMinGroup && a->pf_dist == 0));
-  const bool mfma = mfma_ok && !wave;
+  const bool wave = wave_launch(a);
+  const bool mfma = !wave && mfma_allowed(a);
   if (!mfma && !linear) {
     // VALU K rows are read with 16-byte vector loads.
     if (!aligned16(a->k_pool) || (a->k_tok_stride * eb) % 16 || (a->k_page_stride * eb) % 16 ||
@@ -377,6 +399,8 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = 
                        "the %u tasks", kp->ntasks);
     nsub = a->num_tiles / kp->ntasks;
     kp->sub.pages = a->tile_pages;
+    kp->sub.from =
+        (uint32_t)std::min<uint64_t>(split_from(a, kp->ntasks, a->tile_pages), UINT32_MAX);
   }
   if (a->tiles || split) {
     if (a->tiles && a->tile_format > SCHED_PD_TILES_RANGED)
@@ -779,25 +803,38 @@ int64_t sched_paged_decode_workspace_bytes(const SchedDecodeArgs *a) {
   return (int64_t)ws_layout(a).total;
 }
 
-// When to split (MFMA, bf16, 8 KB a page; whole -> split, us). A launch of few
-// tasks: chunks of kSplitBytes or more of one kv-head's KV, no more items than
-// kFillItems (16 tasks of 257 pages 57 -> 20; below 1.5 chunks a second item
-// costs more than it saves: fp8, 65 pages in chunks of 64, 15 -> 18), and of
-// kHalfFullTokens or more from half the tasks that fill the chip (256 uniform
-// ones of 129 pages in fours: 43 -> 48). From
-// kFullTasks on only contexts of kLongTokens or more, in four (512 ragged tasks
-// of up to 765 pages 163 -> 126, but of up to 383 pages 71 -> 76: their longest
-// items are better whole). With a page list the mean is known, and chunks
-// follow it (512 ragged fp16 tasks of mean 25 pages: 38 -> 34). The one-wave
-// kernel streams an item on one wave, so its chunks are small (128 tasks of
-// mean 18, at most 69 pages: 34 -> 14), larger once the tasks are many (512
-// uniform ones of 17 pages in fifths: 15 -> 17).
-constexpr uint64_t kSplitBytes = 256u << 10, kWaveSplitBytes = 32u << 10;
-constexpr uint64_t kFillItems = 1024, kFullTasks = 512, kWaveFullTasks = 256, kLongTokens = 8192;
-constexpr uint64_t kHalfFullTokens = 1024;
-// Most items of a launch (the empty ones only look at a length), and of a task
-// (its merge reads them all).
-constexpr uint64_t kMostItems = 2048;
+// How a launch without tiles is split: what an item is worth (tile_pages; split_from
+// and item_range make a task's items of it) follows from the number of tasks and a
+// page list's mean, never from a table's width, which only bounds the grid: one
+// request of 8191 tokens takes 16.3 us under tables of 512, 2048 and 8192 pages.
+// Times are in us, MFMA, 16-token pages, whole -> split; the lines come from sweeps
+// over 8..2048 tasks of 200..8192 tokens, of one length and lognormal, with tables 1,
+// 4 and 16 times as wide as the longest and with page lists.
+// - Up to kFewTasks tasks compute units are idle: kSplitBytes of one kv-head's KV (8
+//   bf16 tasks of 513 pages 74 -> 16, at half and twice that 19; 128 of 129 pages 29
+//   -> 27), more where a wide group makes the merge dearer (kSplitBytesWide: 128
+//   fp16 tasks of at most 75 pages, 8 q-heads each, 16.5, with kSplitBytes 18.3).
+// - Below kFullTasks kMidTokens (192 bf16 tasks of mean 123, at most 551 pages: 80 ->
+//   52; 384 at head dim 64, at most 179: 38.8 -> 33.5, at 3/2 of it 41).
+// - Below kOverTasks kFullTokens (512 bf16 tasks of at most 765 pages: 163 -> 126),
+//   from there on kOverTokens, for the longest only.
+// - A page list tells the mean: half of it, all of it at twice the tasks, 5/4 at
+//   most (256 bf16 tasks of mean 136, at most 551: 97 -> 57), for launches that are
+//   worth it (kListBytes; below, 256 tasks of mean 14 pages 13.7 -> 17.1) and leave
+//   the longest four items (kListTasks; 1024 tasks of mean 61 107 -> 121).
+// The one-wave kernel streams an item on one wave: small items (kWaveBytes: 8 fp32
+// tasks of 28 pages 15 -> 8), larger once the tasks fill the chip (kWaveFillBytes: 512
+// tasks 1.2x, with kWaveBytes 0.84x at worst).
+// A merge reads kMergeBatch chunks a round trip: softmax tasks have two of them at
+// most (kMergeChunks; 32 fp16 tasks of at most 551 pages in 17 items 31, in 16 26).
+constexpr uint64_t kSplitBytes = 256u << 10;
+constexpr uint64_t kFullTokens = 3072, kMidTokens = 1024, kOverTokens = 4096;
+constexpr uint64_t kSplitBytesWide = 384u << 10;
+constexpr uint64_t kMergeChunks = 16;
+constexpr uint64_t kListTasks = 512, kListBytes = 64u << 20;
+constexpr uint64_t kWaveFillTasks = 256, kWaveBytes = 32u << 10, kWaveFillBytes = 128u << 10;
+// Most items of a launch (the empty ones only look at a length).
+constexpr uint64_t kMostItems = 2048, kWaveMostItems = 8192;
 
 int64_t sched_paged_decode_auto_split(SchedDecodeArgs *a, uint32_t max_pages,
                                       uint32_t mean_pages) {
@@ -813,35 +850,35 @@ int64_t sched_paged_decode_auto_split(SchedDecodeArgs *a, uint32_t max_pages,
   const uint64_t ntasks = kp.ntasks;
   if (a->tiles || ntasks == 0 || max_pages == 0)
     return 0;
+  const bool wave = sel.mfma == 2;
   const uint64_t page = (uint64_t)a->page_size * a->head_dim * elem_bytes(a->kv_dtype) *
                         (a->mode == SCHED_PD_LINEAR ? 1u : 2u);
-  const bool wave = sel.mfma == 2;
-  auto pages_of = [&](uint64_t bytes) { return std::max<uint64_t>(1u, bytes / page); };
-  const uint64_t per_item = wave ? kWaveSplitBytes * (ntasks >= kWaveFullTasks ? 4u : 1u)
-                                 : kSplitBytes;
-  uint64_t chunk = std::max<uint64_t>(1u, per_item / page);
-  uint64_t s;
-  if (mean_pages) {
-    chunk = std::max(chunk, std::min<uint64_t>(mean_pages + mean_pages / 4u,
-                                               2u * ntasks * mean_pages / kFillItems));
-    s = (max_pages + chunk - 1u) / chunk;
-  } else if (wave) {
-    s = max_pages / std::max(chunk, ntasks * max_pages / (2u * kFillItems));
-  } else if (ntasks < kFullTasks) {
-    if (ntasks >= kFullTasks / 2u)
-      chunk = std::max<uint64_t>(chunk, kHalfFullTokens / a->page_size);
-    chunk = std::max(chunk, ntasks * max_pages / kFillItems);
-    s = (2u * max_pages + chunk) / (2u * chunk);
-  } else {
-    s = (uint64_t)max_pages * a->page_size >= kLongTokens ? 4u : 1u;
-  }
-  s = std::min(std::min(kMostChunks, (wave ? 4u : 1u) * kMostItems / ntasks), s);
-  if (s < 2u)
+  auto of_tokens = [&](uint64_t n) { return n / a->page_size; };
+  // wide groups' merges cost more
+  const uint64_t few = (kp.G > 4u && ntasks <= kFewTasks ? kSplitBytesWide : kSplitBytes) / page;
+  // tasks that fill the chip in one round count as kRoundTasks: half the mean, which
+  // split_from keeps batches of one length whole at
+  const uint64_t list_tasks = ntasks > kFewTasks ? std::max<uint64_t>(ntasks, kRoundTasks) : ntasks;
+  uint64_t least;
+  if (wave)
+    least = (ntasks < kWaveFillTasks ? kWaveBytes : kWaveFillBytes) / page;
+  else if (mean_pages)
+    least = ntasks > kListTasks || (ntasks > kFewTasks && ntasks * mean_pages * page < kListBytes)
+                ? max_pages
+                : std::max(few, std::min<uint64_t>(mean_pages + mean_pages / 4u,
+                                                   list_tasks * mean_pages / kFullTasks));
+  else if (ntasks <= kFewTasks)
+    least = few;
+  else
+    least = of_tokens(ntasks < kFullTasks ? kMidTokens : ntasks < kOverTasks ? kFullTokens : kOverTokens);
+  least = std::max<uint64_t>(1u, least);
+  const uint64_t chunks = wave || a->mode == SCHED_PD_LINEAR ? kMostChunks : kMergeChunks;
+  const uint64_t s = std::min(std::min(chunks, (wave ? kWaveMostItems : kMostItems) / ntasks),
+                              (max_pages + least - 1u) / least);
+  if (s < 2u || max_pages < split_from(a, ntasks, least))
     return 0;
-  if (!mean_pages)
-    chunk = (max_pages + s - 1u) / s;
   a->flags |= SCHED_PD_FLAG_SPLIT;
-  a->tile_pages = (uint32_t)chunk;
+  a->tile_pages = (uint32_t)least;
   a->num_tiles = (uint32_t)(s * ntasks);
   return (int64_t)ws_layout(a).total;
 }

@@ -419,6 +419,7 @@ def _split_on_device(a, block_table, page_indptr, device, stream) -> None:
     if page_indptr is None:
         longest, mean = block_table.shape[1], 0
     else:
+        # the list's length: their total is what is known of the requests
         longest = block_table.numel()
         mean = -(-longest // max(1, a.num_requests))
     need = abi.load_library().sched_paged_decode_auto_split(ctypes.byref(a), longest, mean)

@@ -634,3 +634,23 @@ def test_auto_split_decides_a_refilled_block_afresh(schedlib):
     t = fake_args(tiles=ctypes.c_void_p(0x90000), num_tiles=8, tile_pages=4,
                   workspace=ctypes.c_void_p(0xA0000), workspace_bytes=1 << 20)
     assert split(t, 512) == 0 and (t.num_tiles, t.tile_pages) == (8, 4)
+
+
+@pytest.mark.parametrize("R", [1, 16, 17, 32, 33, 63, 64, 128, 200])
+@pytest.mark.parametrize("kv", [abi.F32, abi.BF16])
+def test_auto_split_does_not_follow_the_table_width(schedlib, R, kv):
+    """A table sized by the model's length cuts the tasks as one that just holds
+    the batch: the same tile_pages, and a grid that holds as many chunks per task,
+    up to the fixed bounds."""
+    got = {}
+    for width in (300, 512, 700, 2048, 8192, 65536):
+        a = fake_args(num_requests=R, num_q_heads=8, num_kv_heads=8, kv_dtype=kv, q_dtype=kv,
+                      v_tok_stride=128, v_dim_stride=1)
+        need = schedlib.sched_paged_decode_auto_split(ctypes.byref(a), width, 0)
+        got[width] = (a.tile_pages, a.num_tiles // (8 * R)) if need > 0 else (0, 1)
+        assert need <= 0 or (a.num_tiles % (8 * R) == 0 and 2 <= got[width][1] <= 32)
+    sizes = {m for m, _ in got.values() if m}
+    # at most 2048 items a launch (8192 of the one-wave kernel's): none for 1600 tasks
+    assert len(sizes) == (1 if 8 * R <= 1024 or kv == abi.F32 else 0)
+    items = [s for _, s in got.values()]
+    assert items == sorted(items) and got[8192] == got[65536]

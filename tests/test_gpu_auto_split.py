@@ -140,6 +140,16 @@ def test_an_order_naming_a_task_twice_leaves_nothing_behind(schedlib, kind):
             assert err.max() <= tol, (workers, shorter, err.max())
 
 
+@pytest.mark.parametrize("kind", ["bf16", "fp8", "wave", "valu"])
+def test_a_wider_table_leaves_the_bits(schedlib, kind):
+    pos, kw, hkv, _ = make(kind)
+    base = run(pos, kw).nan_to_num(9.0)
+    for times in (4, 16):
+        wide = torch.zeros(len(CTX), pos[3].shape[1] * times, dtype=torch.int32, device="cuda")
+        wide[:, :pos[3].shape[1]] = pos[3]
+        assert torch.equal(run((*pos[:3], wide, pos[4]), kw).nan_to_num(9.0), base), times
+
+
 def test_csr_table_and_graph_replays(schedlib):
     pos, kw, hkv, tol = make("bf16")
     base = run(pos, kw).nan_to_num(9.0)
