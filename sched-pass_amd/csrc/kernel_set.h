@@ -75,13 +75,6 @@ constexpr int mfma_du(bool fp8, bool vt, bool pg, bool f16 = false) {
          : (f16 && !pg) ? SCHED_PD_MFMA_DEPTH_F16_URGENT
                         : SCHED_PD_MFMA_DEPTH_URGENT;
 }
-// Lever-free forms: the ring of items longer than kLongItemPages. The linear mode,
-// which holds no K, keeps the lever forms' deep ring for them (16 requests of 6001
-// tokens, 8 heads, bf16: 74.6 -> 49.3 us, the lever form 50.6); the softmax forms'
-// does not fit three waves' registers.
-constexpr int mfma_stock_du(bool fp8, bool vt, bool pg, bool linear) {
-  return linear ? mfma_du(fp8, vt, pg) : mfma_stock(fp8, vt, pg, linear);
-}
 
 } // namespace schedpd
 
@@ -94,8 +87,19 @@ constexpr int mfma_stock_du(bool fp8, bool vt, bool pg, bool linear) {
       schedpd::KParams);                                                                         \
   PRE template __global__ void schedpd::decode_mfma<FP8, SCHED_PD_MFMA_NW, GMAX,                 \
                                                     schedpd::mfma_stock(FP8, VT, PG, LIN),       \
-                                                    schedpd::mfma_stock_du(FP8, VT, PG, LIN),    \
-                                                    LIN, VT, PG, F16, 128, true>(schedpd::KParams);
+                                                    schedpd::mfma_stock(FP8, VT, PG, LIN), LIN,  \
+                                                    VT, PG, F16, 128, true>(schedpd::KParams);
+// Lever-free forms: the ring of items longer than kLongItemPages. The linear mode,
+// which holds no K, has a form with the lever forms' deep ring for launches that may
+// hold such items (long_items; 16 requests of 6001 tokens, 8 heads, bf16: 74.6 -> 49.3
+// us, the lever form 50.6). The others keep the shallow ring and by it a fourth wave
+// per SIMD (1024 tasks of 65 pages 48.3 -> 43.5; 128 of 513 pages in chunks of 64
+// 50.6 -> 44.8). The softmax forms' does not fit three waves' registers.
+#define SCHED_PD_MFMA_LINEAR_DEEP(PRE, FP8, VT, PG)                                              \
+  PRE template __global__ void schedpd::decode_mfma<FP8, SCHED_PD_MFMA_NW, 4,                    \
+                                                    schedpd::mfma_ds(FP8),                       \
+                                                    schedpd::mfma_du(FP8, VT, PG), true, VT, PG, \
+                                                    false, 128, true>(schedpd::KParams);
 #define SCHED_PD_MFMA_SOFTMAX(PRE, FP8, VT, PG, F16)                                             \
   SCHED_PD_MFMA_ONE(PRE, FP8, 4, false, VT, PG, F16)                                             \
   SCHED_PD_MFMA_ONE(PRE, FP8, 8, false, VT, PG, F16)                                             \
@@ -107,13 +111,19 @@ constexpr int mfma_stock_du(bool fp8, bool vt, bool pg, bool linear) {
 // The groups, one per translation unit.
 #define SCHED_PD_MFMA_BF16_PAGE16(PRE)                                                           \
   SCHED_PD_MFMA_WITH_LINEAR(PRE, false, false, false)                                            \
-  SCHED_PD_MFMA_WITH_LINEAR(PRE, false, true, false)
+  SCHED_PD_MFMA_LINEAR_DEEP(PRE, false, false, false)                                            \
+  SCHED_PD_MFMA_WITH_LINEAR(PRE, false, true, false)                                             \
+  SCHED_PD_MFMA_LINEAR_DEEP(PRE, false, true, false)
 #define SCHED_PD_MFMA_BF16_PAGEBLOCKS(PRE)                                                       \
   SCHED_PD_MFMA_WITH_LINEAR(PRE, false, false, true)                                             \
-  SCHED_PD_MFMA_WITH_LINEAR(PRE, false, true, true)
+  SCHED_PD_MFMA_LINEAR_DEEP(PRE, false, false, true)                                             \
+  SCHED_PD_MFMA_WITH_LINEAR(PRE, false, true, true)                                              \
+  SCHED_PD_MFMA_LINEAR_DEEP(PRE, false, true, true)
 #define SCHED_PD_MFMA_FP8(PRE)                                                                   \
   SCHED_PD_MFMA_WITH_LINEAR(PRE, true, false, false)                                             \
-  SCHED_PD_MFMA_WITH_LINEAR(PRE, true, false, true)
+  SCHED_PD_MFMA_LINEAR_DEEP(PRE, true, false, false)                                             \
+  SCHED_PD_MFMA_WITH_LINEAR(PRE, true, false, true)                                              \
+  SCHED_PD_MFMA_LINEAR_DEEP(PRE, true, false, true)
 #define SCHED_PD_MFMA_FP8_TOKMAJOR(PRE)                                                          \
   SCHED_PD_MFMA_WITH_LINEAR(PRE, true, true, false)                                              \
   SCHED_PD_MFMA_WITH_LINEAR(PRE, true, true, true)

@@ -54,14 +54,16 @@ template <typename KVT, int D> KernelFn valu_kernel(bool linear, uint32_t G) {
   return decode_valu<KVT, D, 16, false>;
 }
 
-// `stock`: the launch has no lever tables (decode_mfma's STOCK).
+// `stock`: the launch has no lever tables (decode_mfma's STOCK); `deep`: the linear
+// mode's items may be long.
 template <bool FP8, bool VT = false, bool PG = false>
-KernelFn mfma_kernel(uint32_t G, bool linear, bool stock) {
+KernelFn mfma_kernel(uint32_t G, bool linear, bool stock, bool deep) {
   constexpr int NW = SCHED_PD_MFMA_NW, DS = mfma_ds(FP8), DU = mfma_du(FP8, VT, PG),
-                D0 = mfma_stock(FP8, VT, PG, false), DL = mfma_stock_du(FP8, VT, PG, true);
+                D0 = mfma_stock(FP8, VT, PG, false);
   if (linear)
-    return stock ? decode_mfma<FP8, NW, 4, DS, DL, true, VT, PG, false, 128, true>
-                 : decode_mfma<FP8, NW, 4, DS, DU, true, VT, PG, false>;
+    return !stock ? decode_mfma<FP8, NW, 4, DS, DU, true, VT, PG, false>
+           : deep ? decode_mfma<FP8, NW, 4, DS, DU, true, VT, PG, false, 128, true>
+                  : decode_mfma<FP8, NW, 4, DS, DS, true, VT, PG, false, 128, true>;
   if (stock)
     return G <= 4   ? decode_mfma<FP8, NW, 4, D0, D0, false, VT, PG, false, 128, true>
            : G <= 8 ? decode_mfma<FP8, NW, 8, D0, D0, false, VT, PG, false, 128, true>
@@ -276,6 +278,20 @@ bool stock_launch(const SchedDecodeArgs *a, const KParams &kp) {
          (a->mode == SCHED_PD_LINEAR || (kts >= 0 && kts <= (INT32_MAX - 64) / 16));
 }
 
+// Whether an item of the launch may be longer than kLongItemPages (16-token blocks):
+// a whole task by its table, an item of a split or planned one by what it is worth
+// (ranged rows are cut to the chip, and not).
+bool long_items(const SchedDecodeArgs *a, const KParams &kp) {
+  uint64_t pages = UINT32_MAX;
+  if (a->tiles != nullptr)
+    pages = kp.tile_ranged ? 0u : a->tile_pages;
+  else if (sub_items<true>(kp.L) > 1u)
+    pages = kp.sub.from;
+  else if (a->page_indptr == nullptr)
+    pages = a->bt_stride;
+  return pages * (a->page_size / 16u) > kLongItemPages;
+}
+
 // fp8 token-major V of 16-token pages, softmax: the lever-free form's ring of 3
 // pages and its K exchange make a lone item's stream 5 to 11% slower than the
 // lever form's ring of 4 (one request of 2001 tokens, 8 kv-heads: 22.9 -> 24.6 us;
@@ -476,7 +492,7 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = 
   } else if (mfma) {
     const bool pg = a->page_size > 16;
     const bool stock = !levers && stock_launch(a, *kp) && !lone_fp8_items(a, *kp);
-    const bool vt = v_token_major(a);
+    const bool vt = v_token_major(a), deep = long_items(a, *kp);
     if (a->head_dim == 64)
       sel->fn = a->kv_dtype == SCHED_PD_F16 ? mfma_kernel_d64<true>(G, vt, pg, stock)
                                             : mfma_kernel_d64<false>(G, vt, pg, stock);
@@ -485,16 +501,16 @@ int prepare(const SchedDecodeArgs *a, KParams *kp, Selected *sel, bool levers = 
                    : (pg ? mfma_kernel_f16<false, true>(G, stock)
                          : mfma_kernel_f16<false>(G, stock));
     else if (a->kv_dtype != SCHED_PD_BF16)
-      sel->fn = vt ? (pg ? mfma_kernel<true, true, true>(G, linear, stock)
-                         : mfma_kernel<true, true>(G, linear, stock))
-                : pg ? mfma_kernel<true, false, true>(G, linear, stock)
-                     : mfma_kernel<true>(G, linear, stock);
+      sel->fn = vt ? (pg ? mfma_kernel<true, true, true>(G, linear, stock, deep)
+                         : mfma_kernel<true, true>(G, linear, stock, deep))
+                : pg ? mfma_kernel<true, false, true>(G, linear, stock, deep)
+                     : mfma_kernel<true>(G, linear, stock, deep);
     else if (vt)
-      sel->fn = pg ? mfma_kernel<false, true, true>(G, linear, stock)
-                   : mfma_kernel<false, true>(G, linear, stock);
+      sel->fn = pg ? mfma_kernel<false, true, true>(G, linear, stock, deep)
+                   : mfma_kernel<false, true>(G, linear, stock, deep);
     else
-      sel->fn = pg ? mfma_kernel<false, false, true>(G, linear, stock)
-                   : mfma_kernel<false>(G, linear, stock);
+      sel->fn = pg ? mfma_kernel<false, false, true>(G, linear, stock, deep)
+                   : mfma_kernel<false>(G, linear, stock, deep);
     sel->block = SCHED_PD_MFMA_NW * 64;
     sel->mfma = 1;
   } else {
