@@ -86,7 +86,7 @@ def test_matches_the_oracle_under_every_lever(schedlib, kind):
 
 @pytest.mark.parametrize("kind", list(KINDS))
 def test_shed_budgets_loaded_or_skipped(schedlib, kind):
-    pos, kw, hkv, _ = make(kind)
+    pos, kw, hkv, tol = make(kind)
     n = len(CTX) * hkv
     tau = np.minimum(np.random.default_rng(5).integers(1, 4097, n), 65535)
     outs = []
@@ -96,6 +96,13 @@ def test_shed_budgets_loaded_or_skipped(schedlib, kind):
         plane.push()
         outs.append(run(pos, kw, plane=plane, flags=flags).nan_to_num(9.0))
     assert torch.equal(outs[0], outs[1])
+    live = np.asarray(CTX) > 0
+    ref = np.asarray(oracle.decode(*pos, ctrl=bytes(plane._ctrl_host), max_tasks=n, **kw),
+                     np.float64)[live]
+    got = outs[0].cpu().double().numpy()[live]
+    err = np.linalg.norm(got - ref, axis=-1) / np.linalg.norm(ref, axis=-1)
+    assert err.max() <= tol, err.max()
+    assert not torch.equal(outs[0], run(pos, kw).nan_to_num(9.0))
 
 
 @pytest.mark.parametrize("kind", ["bf16", "wave", "valu"])

@@ -348,6 +348,56 @@ def test_fused_step_under_a_shed_budget(dtype):
             assert same(fa.k_scale, sep.k_scale) and same(fa.v_scale, sep.v_scale), step
 
 
+@pytest.mark.parametrize("kernel", ["mfma", "wave"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, FP8])
+@pytest.mark.parametrize("ps", [16, 64])
+@pytest.mark.parametrize("shed", [False, True])
+def test_fused_step_into_the_later_items_of_a_split_task(kernel, dtype, ps, shed):
+    """Steps that split each task on the device: the token falls into the first,
+    a middle or the last item, on its first or last slot, opens a page there, or
+    (under a budget) lies past every page that is read. Pools, scales and outputs
+    equal append-then-decode, and the oracle under the same budgets."""
+    if kernel == "wave" and dtype == FP8:
+        pytest.skip("no one-wave kernel over fp8 caches")
+    lens = [4999, 639, 640, 1023, 1024, 1279, 2047, 2560, 100]
+    (fa, sep), g = make_pair(dtype, ps, lens, seed=ps + 3)
+    R, G = len(lens), 1 if kernel == "wave" else 4
+    rids = list(range(R))
+    kw = {"flags": abi.FLAG_NO_MFMA} if kernel == "wave" else {}
+    q = (torch.randn(R, HKV * G, D, device="cuda", generator=g) / D ** 0.5).to(qdtype(dtype))
+    if shed:
+        plane = SchedPlane(max_tasks=R * HKV)
+        tau = np.repeat([c // 2 + 1 for c in lens], HKV)
+        tau[::3] = 0                               # no cap: the token's page is read
+        plane.set_rows(tau=tau, n=R * HKV)
+        plane.push()
+        kw["plane"] = plane
+    for step in range(3):
+        amp = 2.0 ** step if dtype == FP8 else 1.0   # fp8: the page re-scales
+        k1 = (torch.randn(R, HKV, D, device="cuda", generator=g) * amp).to(qdtype(dtype))
+        v1 = (torch.randn(R, HKV, D, device="cuda", generator=g) * amp).to(qdtype(dtype))
+        if shed and step == 2:
+            kw["flags"] = kw.get("flags", 0) | abi.FLAG_SHED_LOADS
+        o_fused = fa.decode_step(q, rids, k1, v1, out_dtype=torch.float32, **kw)
+        sep.append(rids, k1, v1)
+        o_sep = sep.decode(q, rids, out_dtype=torch.float32, **kw)
+        torch.cuda.synchronize()
+        assert same(fa.k_pool, sep.k_pool) and same(fa.v_pool, sep.v_pool), step
+        if dtype == FP8:
+            assert same(fa.k_scale, sep.k_scale) and same(fa.v_scale, sep.v_scale), step
+        assert same(o_fused, o_sep), step
+    bt, ctx = fa.block_table(rids)
+    a = sched_pd.build_args(q, fa.k_pool, fa.v_pool, bt, ctx, out=o_fused, v_layout="tokmajor",
+                            k_scale=fa.k_scale, v_scale=fa.v_scale, **kw)
+    assert sched_pd.kernel_kind(a) == kernel
+    assert abi.load_library().sched_paged_decode_auto_split(a, bt.shape[1], 0) > 0
+    assert a.tile_pages * ps <= 1024               # 4999 tokens: four items or more
+    ref = oracle.decode(q, fa.k_pool, fa.v_pool, bt, ctx, v_layout="tokmajor",
+                        k_scale=fa.k_scale, v_scale=fa.v_scale,
+                        **({"ctrl": bytes(plane._ctrl_host), "max_tasks": R * HKV} if shed else {}))
+    assert par_err(o_fused.cpu(), ref, f"split {kernel} {dtype} p{ps}") <= TOL_BF16
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, FP8])
 @pytest.mark.parametrize("G", [1, 4])
 def test_fused_step_opens_an_empty_requests_first_page(dtype, G):
