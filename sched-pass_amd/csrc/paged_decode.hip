@@ -306,24 +306,28 @@ bool lone_fp8_items(const SchedDecodeArgs *a, const KParams &kp) {
   if (a->kv_dtype != SCHED_PD_FP8_E4M3 || a->mode == SCHED_PD_LINEAR || !v_token_major(a) ||
       a->page_size != 16 || kp.L.nitems > kLoneItems)
     return false;
-  if (a->tiles != nullptr)
-    return kp.tile_ranged || a->tile_pages > kLoneItemPages;
-  return sub_items<true>(kp.L) > 1u || a->page_indptr != nullptr || a->bt_stride > kLoneItemPages;
+  return (a->page_indptr != nullptr || a->bt_stride > kLoneItemPages) &&
+         (a->tiles == nullptr || kp.tile_ranged || a->tile_pages > kLoneItemPages);
 }
 
 // Task counts between which the split's rule changes (sched_paged_decode_auto_split).
-constexpr uint32_t kFewTasks = 128, kRoundTasks = 256, kFullTasks = 512, kOverTasks = 1024;
+// kRoundTasks: a workgroup per CU. kHalfTasks: two items of each are the three
+// workgroups per CU that the lever-free forms hold at once.
+constexpr uint32_t kFewTasks = 128, kRoundTasks = 256, kHalfTasks = 384, kFullTasks = 512,
+                   kOverTasks = 1024;
 
 // Pages from which a split launch splits a task, where an item is worth `least`:
-// 5/4 of it, but 5/2 where the tasks are a workgroup per CU or nearly, or two and
-// more, and tasks of one length keep every CU busy by themselves and in two items
-// only pay for the merge (192 fp8 tasks of 129 pages: 20.5 us whole, 25.8 in two;
-// 256 bf16 ones 43 and 47; 512 of mean 70, at most 383: 71 and 87); a page list's
-// mean keeps full launches whole by itself. The one-wave kernel's small items: twice
-// (8 fp32 tasks of 6 pages: 6.7 whole, 8.2 in two).
+// 5/4 of it, but 5/2 where tasks of one length keep every CU busy by themselves and
+// in two items only pay for the merge: a workgroup per CU or nearly (192 fp8 tasks of
+// 129 pages: 20.5 us whole, 25.8 in two; 256 bf16 ones 43 and 47), and past
+// kHalfTasks, where their second items wait for a second round (fp8, 129 pages: 384
+// tasks 38.6 and 39.6, 400 tasks 38.9 and 46.5; bf16 67.1 and 68.7, 68.0 and 79.0; 512
+// of mean 70, at most 383: 71 and 87). There a page list's mean keeps batches of one
+// length whole by itself. The one-wave kernel's small items: twice (8 fp32 tasks of 6
+// pages: 6.7 whole, 8.2 in two).
 uint64_t split_from(const SchedDecodeArgs *a, uint64_t ntasks, uint64_t least) {
   const bool full = ntasks > kFewTasks && (ntasks <= kRoundTasks ||
-                                           (ntasks >= kFullTasks && a->page_indptr == nullptr));
+                                           (ntasks > kHalfTasks && a->page_indptr == nullptr));
   return least * (wave_launch(a) ? 8u : full ? 10u : 5u) / 4u;
 }
 
@@ -822,32 +826,34 @@ int64_t sched_paged_decode_workspace_bytes(const SchedDecodeArgs *a) {
 // How a launch without tiles is split: what an item is worth (tile_pages; split_from
 // and item_range make a task's items of it) follows from the number of tasks and a
 // page list's mean, never from a table's width, which only bounds the grid: one
-// request of 8191 tokens takes 16.3 us under tables of 512, 2048 and 8192 pages.
+// request of 8193 tokens takes 16.6 us under tables of 513, 2052 and 8208 pages.
 // Times are in us, MFMA, 16-token pages, whole -> split; the lines come from sweeps
 // over 8..2048 tasks of 200..8192 tokens, of one length and lognormal, with tables 1,
 // 4 and 16 times as wide as the longest and with page lists.
 // - Up to kFewTasks tasks compute units are idle: kSplitBytes of one kv-head's KV (8
-//   bf16 tasks of 513 pages 74 -> 16, at half and twice that 19; 128 of 129 pages 29
-//   -> 27), more where a wide group makes the merge dearer (kSplitBytesWide: 128
-//   fp16 tasks of at most 75 pages, 8 q-heads each, 16.5, with kSplitBytes 18.3).
-// - Below kFullTasks kMidTokens (192 bf16 tasks of mean 123, at most 551 pages: 80 ->
-//   52; 384 at head dim 64, at most 179: 38.8 -> 33.5, at 3/2 of it 41).
-// - Below kOverTasks kFullTokens (512 bf16 tasks of at most 765 pages: 163 -> 126),
+//   bf16 tasks of 513 pages 74 -> 16.6, at half and twice that 19; 128 of 129 pages
+//   28.8 -> 27.9), more where a wide group makes the merge dearer (kSplitBytesWide: 128
+//   fp16 tasks of at most 75 pages, 8 q-heads each, 16.7 -> 17.4, with kSplitBytes
+//   18.3; at most 383 pages 56.1 -> 34.4).
+// - Below kFullTasks kMidTokens (192 bf16 tasks of mean 123, at most 551 pages: 81 ->
+//   51; 384 at head dim 64, at most 179: 38.8 -> 33.5, at 3/2 of it 41).
+// - Below kOverTasks kFullTokens (512 fp8 tasks of mean 139, at most 765 pages: 105 -> 74),
 //   from there on kOverTokens, for the longest only.
 // - A page list tells the mean: half of it, all of it at twice the tasks, 5/4 at
-//   most (256 bf16 tasks of mean 136, at most 551: 97 -> 57), for launches that are
+//   most (256 bf16 tasks of mean 136, at most 551: 97 -> 65), for launches that are
 //   worth it (kListBytes; below, 256 tasks of mean 14 pages 13.7 -> 17.1) and leave
 //   the longest four items (kListTasks; 1024 tasks of mean 61 107 -> 121).
 // The one-wave kernel streams an item on one wave: small items (kWaveBytes: 8 fp32
-// tasks of 28 pages 15 -> 8), larger once the tasks fill the chip (kWaveFillBytes: 512
-// tasks 1.2x, with kWaveBytes 0.84x at worst).
+// tasks of 28 pages 15.2 -> 8.5), larger once the tasks fill the chip (kWaveFillBytes: 512
+// of at most 75 pages 37.8 -> 21.1; 512 of 13 with kWaveBytes 0.84x).
 // A merge reads kMergeBatch chunks a round trip: softmax tasks have two of them at
-// most (kMergeChunks; 32 fp16 tasks of at most 551 pages in 17 items 31, in 16 26).
+// most (kMergeChunks; 32 fp16 tasks of at most 551 pages in up to 17 items of 32 31.1,
+// in up to 16 26.0).
 constexpr uint64_t kSplitBytes = 256u << 10;
 constexpr uint64_t kFullTokens = 3072, kMidTokens = 1024, kOverTokens = 4096;
 constexpr uint64_t kSplitBytesWide = 384u << 10;
 constexpr uint64_t kMergeChunks = 16;
-constexpr uint64_t kListTasks = 512, kListBytes = 64u << 20;
+constexpr uint64_t kListTasks = 512, kListFullTasks = 440, kListBytes = 64u << 20;
 constexpr uint64_t kWaveFillTasks = 256, kWaveBytes = 32u << 10, kWaveFillBytes = 128u << 10;
 // Most items of a launch (the empty ones only look at a length).
 constexpr uint64_t kMostItems = 2048, kWaveMostItems = 8192;
@@ -872,9 +878,11 @@ int64_t sched_paged_decode_auto_split(SchedDecodeArgs *a, uint32_t max_pages,
   auto of_tokens = [&](uint64_t n) { return n / a->page_size; };
   // wide groups' merges cost more
   const uint64_t few = (kp.G > 4u && ntasks <= kFewTasks ? kSplitBytesWide : kSplitBytes) / page;
-  // tasks that fill the chip in one round count as kRoundTasks: half the mean, which
-  // split_from keeps batches of one length whole at
-  const uint64_t list_tasks = ntasks > kFewTasks ? std::max<uint64_t>(ntasks, kRoundTasks) : ntasks;
+  // tasks that fill the chip in one round count as kRoundTasks: half the mean, at
+  // which split_from keeps batches of one length whole; past kHalfTasks 6/7 of it
+  const uint64_t list_tasks = ntasks > kHalfTasks ? std::max<uint64_t>(ntasks, kListFullTasks)
+                              : ntasks > kFewTasks ? std::max<uint64_t>(ntasks, kRoundTasks)
+                                                   : ntasks;
   uint64_t least;
   if (wave)
     least = (ntasks < kWaveFillTasks ? kWaveBytes : kWaveFillBytes) / page;

@@ -445,10 +445,15 @@ def _split_on_device(a, block_table, page_indptr, device, stream) -> None:
 
 def _in_private_pool(t) -> bool:
     """Whether the caching allocator took `t` from a graph's (or MemPool's) own
-    pool; memory of the ordinary pool goes to other tensors once `t` is dropped."""
+    pool; memory of the ordinary pool goes to other tensors once `t` is dropped.
+    An allocator that cannot tell has no such pool."""
     p = t.data_ptr()
+    try:
+        segments = torch.cuda.memory_snapshot()
+    except RuntimeError:
+        return False
     return any(s["address"] <= p < s["address"] + s["total_size"]
-               and tuple(s["segment_pool_id"]) != (0, 0) for s in torch.cuda.memory_snapshot())
+               and tuple(s["segment_pool_id"]) != (0, 0) for s in segments)
 
 
 _WS = {}
