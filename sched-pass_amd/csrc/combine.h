@@ -302,9 +302,11 @@ __device__ __forceinline__ ItemRange item_range(const KParams &P, const ItemRow 
     it.nchunks = 1u;
     if (pages >= P.sub.from) { // a task too short pays for no division
       const uint32_t nsub = sub_items<SPLIT>(P.L);
-      it.cp = max(m, (pages + nsub - 1u) / nsub);
+      it.cp = pages > m * nsub ? (pages + nsub - 1u) / nsub : m;
       nc = (4u * pages + 3u * it.cp) / (4u * it.cp);
-      it.nchunks = min(nc, max(1u, (npages_load + it.cp - 1u) / it.cp));
+      it.nchunks = npages_load >= pages
+                       ? nc
+                       : min(nc, max(1u, (npages_load + it.cp - 1u) / it.cp));
     }
     it.p0 = min(I.chunk * it.cp, npages_load);
     it.p1 = I.chunk + 1u < nc ? min(it.p0 + it.cp, npages_load) : npages_load;

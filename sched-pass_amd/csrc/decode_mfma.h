@@ -37,7 +37,7 @@
 // tokens is selected to 0 (mask_v64: gqa d64 step 34.6 -> 34.9 us). HBM-bound as
 // head dim 128 is, at half the bytes per page, so the ring holds twice the
 // pages: 48 requests of 200..2900 tokens, 32 / 8 heads, bf16: 170 us on the
-// VALU kernel, 38 us here (34 split on the device, 4.7 TB/s), with an
+// VALU kernel, 38 us here (33.5 split on the device, 4.8 TB/s), with an
 // fp32 output's error against 64 bits at 2.3e-7 (VALU: 3.4e-7).
 //
 // Pages of 32..256 tokens (PG): the kernel streams 16-token blocks; block b
