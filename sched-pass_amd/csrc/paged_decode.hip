@@ -323,12 +323,17 @@ constexpr uint32_t kFewTasks = 128, kRoundTasks = 256, kHalfTasks = 384, kFullTa
 // kHalfTasks, where their second items wait for a second round (fp8, 129 pages: 384
 // tasks 38.6 and 39.6, 400 tasks 38.9 and 46.5; bf16 67.1 and 68.7, 68.0 and 79.0; 512
 // of mean 70, at most 383: 71 and 87). There a page list's mean keeps batches of one
-// length whole by itself. The one-wave kernel's small items: twice (8 fp32 tasks of 6
-// pages: 6.7 whole, 8.2 in two).
+// length whole by itself. Twice an item's worth for the one-wave kernel's small items
+// (8 fp32 tasks of 6 pages: 6.7 whole, 8.2 in two); 7/4 for few softmax tasks on the
+// matrix cores, where less is over before the host's next call (8 fp16 tasks of 39 to
+// 78 pages, the call: 14.4 whole, 16.1 split; the linear mode's half bytes make longer
+// items: 44 fp8 tasks of up to 246 pages 22.5 with 5/4, 33.9 with 7/4).
 uint64_t split_from(const SchedDecodeArgs *a, uint64_t ntasks, uint64_t least) {
   const bool full = ntasks > kFewTasks && (ntasks <= kRoundTasks ||
                                            (ntasks > kHalfTasks && a->page_indptr == nullptr));
-  return least * (wave_launch(a) ? 8u : full ? 10u : 5u) / 4u;
+  const bool few =
+      ntasks <= kFewTasks && a->mode == SCHED_PD_SOFTMAX && mfma_allowed(a);
+  return least * (wave_launch(a) ? 8u : few ? 7u : full ? 10u : 5u) / 4u;
 }
 
 // Validate `a`; on success fill *kp (tables resolved) and *sel (`levers`: the
